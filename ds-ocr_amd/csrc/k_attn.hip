@@ -2,45 +2,71 @@
 // ds_moe_decoder.c:339-431; MHA, single-token decode) on the device:
 //   k_attn_qkv     : x_norm = ds_rms_norm(x) in its AVX-512 order (recomputed by every block), then
 //                    the rows of [Wq; Wk; Wv] in ds_linear_nobias_bf16_qkv's AVX-512 order with its
-//                    split of the rows over the reference's threads (ds_kernels.c:844-915); v goes
-//                    straight into the V cache row pos;
-//   k_attn_scores  : per head x chunk of positions, the optional per-head q/k norms and RoPE
-//                    (ds_apply_rope_neox, recomputed by every block), the roped k into the K cache row
-//                    pos, and the scores;
-//   k_attn_coef, k_attn_av, k_attn_combine : the online-softmax attention over the causal or R-SWA
-//                    positions (below), spread over heads x position chunks;
-//   k_attn_oproj   : proj = Wo·att in ds_bf16_matvec_threaded's order;
+//                    split of the rows over the reference's threads (ds_kernels.c:844-915), RoPE
+//                    (ds_apply_rope_neox) on the q and k rows; k and v go straight into the cache rows pos;
+//   k_attn_scores  : per head x chunk of positions the scores and their maximum (with per-head q/k
+//                    norms also the norms and RoPE, recomputed by every block);
+//   k_attn_av      : per head x chunk the online softmax's coefficients over the causal or R-SWA
+//                    positions (below) and the chunk's sum of V rows;
+//   k_attn_oproj   : the chunks' sums put together, then proj = Wo·att in ds_bf16_matvec_threaded's
+//                    order;
 //   k_attn_post    : h = x + proj and n = ds_rms_norm(h) (ds_residual_rms_norm, AVX-512 order).
+// A token moves 13 MB of projections and 10 KB per cached position, a few microseconds of HBM time: what
+// bounds it is the number of dependent launches (about 2 us each) and the latency inside each of them.
 // Everything except the attention's output sum is bit-exact with the reference. The reference's
 // attention is a sequential online softmax with ds_fast_expf (ds_kernels.c:2124-2160,
 // :2270-2330). Its branch at each position depends only on the running maximum, so these kernels
 // take the same branches with the same exp arguments: a prefix-max scan gives each position's
 // running maximum P, its factor f = fast_exp(P - s) on a new maximum (the correction) or
 // fast_exp(s - P) (its weight), and a suffix product of the later corrections gives each V row's
-// final coefficient c; o = sum c*v and sum_e = sum c are then sums in any order. The result differs
-// from the reference's sequential recurrence by f32 rounding only.
+// final coefficient c; o = sum c*v and sum_e = sum c are then sums in any order. A chunk of positions
+// needs the maximum of the positions before it (the chunk maxima that k_attn_scores leaves) and
+// hands on its product of corrections, by which the chunks before it are scaled when the sums are
+// put together. The result differs from the reference's sequential recurrence by f32 rounding only.
 #include "dsh.h"
 #include "dsh_avx.h"
 #include "k_core.h"
 
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+
 __device__ __forceinline__ int attn_pos(const int *pos_ptr, int pos_add) { return (pos_ptr ? *pos_ptr : 0) + pos_add; }
 
-// ds_rms_norm's sum of squares (AVX-512 branch): 16 lanes of fused squares over n/16 steps, then
-// the reduce tree. Called by all threads; x in LDS, n % 16 == 0. Returns r = 1/sqrtf(sum/n + eps)
-// to every thread (s_r: one LDS float).
-__device__ float attn_rms_scale(const float *x, int n, float eps, float *s_r) {
-  if (threadIdx.x < 16) {
-    float acc = 0.0f;
-    for (int i = 0; i < n; i += 16) acc = __builtin_fmaf(x[i + threadIdx.x], x[i + threadIdx.x], acc);
-    // tree16: T3[i] = A[8+i] + A[i]; T6[j] = T3[4+j] + T3[j]; (T6[0]+T6[2]) + (T6[1]+T6[3])
-    const float t3 = __shfl_down(acc, 8, 16) + acc;
-    const float t6 = __shfl_down(t3, 4, 16) + t3;
-    const float t02 = __shfl_down(t6, 2, 16) + t6;  // lane 0: T6[0]+T6[2]; lane 1: T6[1]+T6[3]
-    const float s = t02 + __shfl_down(t02, 1, 16);
-    if (threadIdx.x == 0) *s_r = 1.0f / __builtin_sqrtf(s / (float)n + eps);
+// Sum over each aligned group of 16 lanes in _mm512_reduce_add_ps's tree (GCC 11): T3[i] = A[8+i] + A[i],
+// T6[j] = T3[4+j] + T3[j], (T6[0]+T6[2]) + (T6[1]+T6[3]), lane i holding A[i]. f32 addition commutes,
+// so every lane of the group gets the sum's bits; after a step the values repeat, which lets a
+// rotation by 4 stand for the exchange with lane ^ 4.
+__device__ __forceinline__ float attn_tree16(float v) {
+  v += dsh_dpp<0x128>(v);  // row_ror:8
+  v += dsh_dpp<0x124>(v);  // row_ror:4
+  v += dsh_dpp<0x4E>(v);   // quad_perm [2,3,0,1]
+  return v + dsh_dpp<0xB1>(v);
+}
+
+// ds_rms_norm's scale (AVX-512 branch): 16 chains of fused squares over n/16 steps, then the tree;
+// r = 1/sqrtf(sum/n + eps). Every 16-lane row of every wave computes it (no barrier, no broadcast
+// through LDS). x in LDS, n % 16 == 0. All of a lane's LDS reads are issued ahead of its chain of dependent
+// steps (read as needed, three at a time, the chain waited for each).
+template <int N>
+struct attn_rms {
+  float v[N / 16];
+  __device__ __forceinline__ void read(const float *x) {
+#pragma unroll
+    for (int i = 0; i < N / 16; i++) v[i] = x[16 * i + (threadIdx.x & 15)];
   }
-  __syncthreads();
-  return *s_r;
+  __device__ __forceinline__ float scale(float eps) const {
+    float acc = 0.0f;
+#pragma unroll
+    for (int i = 0; i < N / 16; i++) acc = __builtin_fmaf(v[i], v[i], acc);
+    return 1.0f / __builtin_sqrtf(attn_tree16(acc) / (float)N + eps);
+  }
+};
+
+template <int N>
+__device__ __forceinline__ float attn_rms_scale(const float *x, float eps) {
+  attn_rms<N> r;
+  r.read(x);
+  __builtin_amdgcn_sched_barrier(0);
+  return r.scale(eps);
 }
 
 // Path of global row R of [q; k; v] under ds_linear_nobias_bf16_qkv's split: thread t takes rows
@@ -62,147 +88,176 @@ __device__ __forceinline__ int qkv_row_path(int R, int q_dim, int kv_dim, int nt
   return off < (len & ~1) ? DSH_ROW_GROUP2 : DSH_ROW_SINGLE;
 }
 
-// One bf16 row of length 32*N32 against x (LDS) at lane L of its 4-lane group, in the path's order.
+// A bf16 row of length 32*N32 by a 16-lane group, 4 bytes per lane and load: lane c holds columns
+// 32i + 2c and 32i + 2c + 1 (c < 8: the reference's accumulator a0, else a1). Sixteen lanes to a row (not
+// four with 16-byte loads) give a projection of 1280 x 1280 to 4 waves on each of 80 CUs and leave a lane two
+// chains of N32 steps instead of eight.
 template <int N32>
-__device__ __forceinline__ float attn_row(const uint16_t *w, const u32x4 *wv, const float *x, int L, int path) {
-  if (path == DSH_ROW_SINGLE) return avx_row<true>(w, x, 32 * N32, L, true, true, 0.0f, true);
-  return avx_row_regs32<N32>(wv, x, L, true, 0.0f);
+__device__ __forceinline__ void attn_row_load(uint32_t *wv, const uint16_t *w, int c) {
+#pragma unroll
+  for (int i = 0; i < N32; i++) wv[i] = ((const uint32_t *)w)[16 * i + c];
 }
 
-// Every lane's 16-byte pieces of its row (columns 32i + 8L .. +7), issued together.
+// The lane's columns of x (LDS), read ahead of their use.
 template <int N32>
-__device__ __forceinline__ void attn_row_load(u32x4 *wv, const uint16_t *w, int L) {
+__device__ __forceinline__ void attn_row_x(f32x2 *xv, const float *x, int c) {
 #pragma unroll
-  for (int i = 0; i < N32; i++) wv[i] = ((const u32x4 *)w)[4 * i + L];
+  for (int i = 0; i < N32; i++) xv[i] = ((const f32x2 *)x)[16 * i + c];
+}
+
+// The row's value (all 16 lanes) in the path's order against x[k] * rs (rounded; SCALE false: x[k]); xv: the
+// lane's columns of x, x in LDS for single rows. The 4- and 2-row groups run 32 chains (a0, a1), then
+// a0 + a1 and the tree; a single row 16 chains over 16-column steps. Then "+ bias", 0.0f when absent
+// (ds_kernels_avx.c:84-87).
+template <int N32, bool SCALE>
+__device__ __forceinline__ float attn_row(const uint16_t *w, const uint32_t *wv, const f32x2 *xv, const float *x,
+                                          float rs, int c, int path) {
+  if (path == DSH_ROW_SINGLE) {
+    float a = 0.0f;
+    for (int i = 0; i < 2 * N32; i++) {
+      const float xs = x[16 * i + c];
+      a = __builtin_fmaf(dsh_bf16_to_f32(w[16 * i + c]), SCALE ? xs * rs : xs, a);
+    }
+    return attn_tree16(a) + 0.0f;
+  }
+  float a0 = 0.0f, a1 = 0.0f;
+#pragma unroll
+  for (int i = 0; i < N32; i++) {
+    a0 = __builtin_fmaf(dsh_bf16lo(wv[i]), SCALE ? xv[i][0] * rs : xv[i][0], a0);
+    a1 = __builtin_fmaf(dsh_bf16hi(wv[i]), SCALE ? xv[i][1] * rs : xv[i][1], a1);
+  }
+  // lane c: chains 2c and 2c+1; a0 + a1 adds lanes c and c + 8, then the tree over pairs of columns
+  f32x2 v = {a0, a1};
+  v[0] += dsh_dpp<0x128>(v[0]);
+  v[1] += dsh_dpp<0x128>(v[1]);
+  v[0] += dsh_dpp<0x124>(v[0]);  // T3: columns 8+i and i are lanes c + 4 and c
+  v[1] += dsh_dpp<0x124>(v[1]);
+  v[0] += dsh_dpp<0x4E>(v[0]);  // T6: lanes c + 2 and c
+  v[1] += dsh_dpp<0x4E>(v[1]);
+  v[0] += dsh_dpp<0xB1>(v[0]);  // T6[0]+T6[2] and T6[1]+T6[3]
+  v[1] += dsh_dpp<0xB1>(v[1]);
+  return (v[0] + v[1]) + 0.0f;
 }
 
 // ---------------------------------------------------------------------------- QKV
-// 64 rows of [q; k; v] per 256-thread block (4 lanes per row). H == 32*N32.
-// Pieces i0 and i1 (f32x4; i1 < 0: none) of x into LDS dst, x summed over ncopies (1 or 8) copies
-// [ncopies][H] in copy order; every load is issued before the first add. Also to x_out when given.
-__device__ __forceinline__ void attn_x_pieces(const float *x, int H, int ncopies, int i0, int i1, float *dst,
-                                              float *x_out) {
-  const f32x4 *x4 = (const f32x4 *)x;
-  const int H4 = H / 4, j0 = i0 < 0 ? 0 : i0, j1 = i1 < 0 ? j0 : i1;
-  f32x4 a = x4[j0], b = x4[j1];
-  if (ncopies == 8) {
-    f32x4 ca[7], cb[7];
+// The input vector x (H floats, H % 256 == 0), summed over NC (1 or 8) copies [NC][H] in copy order, by a
+// block of TH threads: a thread holds the f32x4 pieces threadIdx.x + TH * k (past the end it repeats the
+// last one, so that the loads stay unconditional and the waits for them counted). load() issues every load,
+// so that a kernel can issue its rows behind them; the adds and stores come with store().
+template <int H, int NC, int TH>
+struct attn_x {
+  static constexpr int NK = (H / 4 + TH - 1) / TH;
+  f32x4 v[NC][NK], w[NK];
+  static __device__ __forceinline__ int piece(int k) { return min((int)threadIdx.x + TH * k, H / 4 - 1); }
+  __device__ __forceinline__ void load(const float *x, const float *wn) {
 #pragma unroll
-    for (int c = 0; c < 7; c++) {
-      ca[c] = x4[(size_t)(c + 1) * H4 + j0];
-      cb[c] = x4[(size_t)(c + 1) * H4 + j1];
-    }
+    for (int k = 0; k < NK; k++) {
 #pragma unroll
-    for (int c = 0; c < 7; c++) {
-      a += ca[c];
-      b += cb[c];
+      for (int c = 0; c < NC; c++) v[c][k] = ((const f32x4 *)x)[(size_t)c * (H / 4) + piece(k)];
+      if (wn) w[k] = ((const f32x4 *)wn)[piece(k)];
     }
   }
-  if (i0 >= 0) {
-    ((f32x4 *)dst)[i0] = a;
-    if (x_out) ((f32x4 *)x_out)[i0] = a;
+  // x to dst (LDS) and x_out (if given), x times the norm's weights to dst_w (if given)
+  __device__ __forceinline__ void store(float *dst, float *dst_w, float *x_out) {
+#pragma unroll
+    for (int k = 0; k < NK; k++) {
+      f32x4 a = v[0][k];
+#pragma unroll
+      for (int c = 1; c < NC; c++) a += v[c][k];
+      if ((int)threadIdx.x + TH * k >= H / 4) continue;
+      ((f32x4 *)dst)[piece(k)] = a;
+      if (dst_w) ((f32x4 *)dst_w)[piece(k)] = a * w[k];
+      if (x_out) ((f32x4 *)x_out)[piece(k)] = a;
+    }
   }
-  if (i1 >= 0) {
-    ((f32x4 *)dst)[i1] = b;
-    if (x_out) ((f32x4 *)x_out)[i1] = b;
-  }
-}
+};
+// Threads of a block that puts n floats together, one f32x4 each.
+__host__ __device__ constexpr int attn_threads(int n) { return n / 4 > 256 ? n / 4 : 256; }
 
-template <int N32>
+// 16 rows of one of q, k, v per 256-thread block (16 lanes per row): 240 blocks at 1280 x 1280, about one
+// per CU, each with 40 KB of rows in flight behind its input. The rows of a q or k block are eight
+// (d, d + head_dim/2) pairs of one head, a pair in one wave, so the block applies RoPE itself (without the per-head
+// norms, which need the whole head first: then q and k go out as they are, for k_attn_scores). 5.5 us at
+// 1280 x 1280 (9.8 MB, half of it launch and the input's round trip) against 8.1 with 64 rows per block on 60 CUs.
+// H == 32*N32; head_dim % 16 == 0.
+template <int N32, int NC>
 __global__ void __launch_bounds__(256) k_attn_qkv(dsh_attn_t A, const float *x_in, const int *step, int stride,
-                                                  int ncopies, float *x_plain, const int *pos_ptr, int pos_add,
+                                                  float *x_plain, const int *pos_ptr, int pos_add,
                                                   int nthreads) {
   constexpr int H = 32 * N32;
-  __shared__ __attribute__((aligned(16))) float s_x[H];
-  __shared__ float s_r;
-  const int qd = A.n_heads * A.head_dim, total = 3 * qd;
-  const int L = threadIdx.x & 3;
-  const int R = blockIdx.x * 64 + (threadIdx.x >> 2);
-  const int Rc = R < total ? R : total - 1;
-  const int m = Rc < qd ? 0 : (Rc < 2 * qd ? 1 : 2), r = Rc - m * qd;
+  __shared__ __attribute__((aligned(16))) float s_x[H], s_xw[H];
+  const int hd = A.head_dim, half = hd / 2, qd = A.n_heads * hd, bpm = qd / 16, bph = hd / 16;
+  const int m = blockIdx.x / bpm, b = blockIdx.x - m * bpm;
+  const int c = threadIdx.x & 15, slot = (threadIdx.x >> 4) & 3, wave = threadIdx.x >> 6;
+  const int h = b / bph, t = 8 * (b - h * bph) + 2 * wave + (slot & 1) + (slot >> 1) * half;  // q, k
+  const int r = m == 2 ? 16 * b + 4 * wave + slot : h * hd + t;
   const uint16_t *w = (m == 0 ? A.wq : (m == 1 ? A.wk : A.wv)) + (size_t)r * H;
-  const int path = qkv_row_path(Rc, qd, qd, nthreads);
-  u32x4 wv[N32];
-  if (path != DSH_ROW_SINGLE) attn_row_load<N32>(wv, w, L);
+  const int path = qkv_row_path(m * qd + r, qd, qd, nthreads);
+  const int pos = attn_pos(pos_ptr, pos_add);
   const float *x = step ? x_in + (size_t)(*step) * stride : x_in;
-  // H/4 <= 512 pieces: at most two per thread (block 0 also writes x for the residual kernel)
-  attn_x_pieces(x, H, ncopies, (int)threadIdx.x < H / 4 ? (int)threadIdx.x : -1,
-                (int)threadIdx.x + 256 < H / 4 ? (int)threadIdx.x + 256 : -1, s_x, blockIdx.x == 0 ? x_plain : nullptr);
-  __syncthreads();
-  const float rs = attn_rms_scale(s_x, H, A.eps, &s_r);
-  float xn[(H + 255) / 256];
-#pragma unroll
-  for (int k = 0; k < (H + 255) / 256; k++) {
-    const int i = threadIdx.x + 256 * k;
-    if (i < H) xn[k] = (s_x[i] * A.in_norm[i]) * rs;
+  attn_x<H, NC, 256> X;
+  X.load(x, A.in_norm);
+  uint32_t wv[N32];
+  float cs = 0.0f, sn = 0.0f;
+  attn_row_load<N32>(wv, w, c);
+  if (m != 2) {
+    cs = A.rope_cos[(size_t)pos * hd + t];
+    sn = A.rope_sin[(size_t)pos * hd + t];
   }
-  __syncthreads();  // every thread has read s_x
-#pragma unroll
-  for (int k = 0; k < (H + 255) / 256; k++) {
-    const int i = threadIdx.x + 256 * k;
-    if (i < H) s_x[i] = xn[k];
-  }
+  __builtin_amdgcn_sched_barrier(0);  // every load is on its way before the first wait
+  X.store(s_x, s_xw, blockIdx.x == 0 ? x_plain : nullptr);  // block 0: x for the residual kernel
   __syncthreads();
-  const float v = attn_row<N32>(w, wv, s_x, L, path);
-  if (L == 0 && R < total) {
+  attn_rms<H> rms;
+  f32x2 xv[N32];
+  rms.read(s_x);
+  attn_row_x<N32>(xv, s_xw, c);
+  __builtin_amdgcn_sched_barrier(0);
+  const float rs = rms.scale(A.eps);
+  float v = attn_row<N32, true>(w, wv, xv, s_xw, rs, c, path);
+  if (m == 2) {
+    if (c == 0) A.vc[(size_t)pos * A.kv_stride + r] = v;
+    return;
+  }
+  if (A.q_norm || A.k_norm) {
+    if (c == 0) (m == 0 ? A.q : A.k)[r] = v;
+    return;
+  }
+  const float u = __shfl_xor(v, 32);  // the pair's other row
+  v = slot < 2 ? __builtin_fmaf(v, cs, -(u * sn)) : __builtin_fmaf(u, sn, v * cs);
+  if (c == 0) {
     if (m == 0)
       A.q[r] = v;
-    else if (m == 1)
-      A.k[r] = v;
     else
-      A.vc[(size_t)attn_pos(pos_ptr, pos_add) * A.kv_stride + r] = v;
+      A.kc[(size_t)pos * A.kv_stride + r] = v;
   }
 }
 
 // ---------------------------------------------------------------------------- attention core
-#define ATTN_THREADS 256
-
-// Inclusive scan over the block's threads (ATTN_THREADS) with an associative op; s_w: 4 floats.
-template <typename Op>
-__device__ __forceinline__ float attn_block_scan(float v, Op op, float *s_w) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const float u = __shfl_up(v, o);
-    if (lane >= o) v = op(u, v);
-  }
-  if (lane == 63) s_w[wave] = v;
-  __syncthreads();
-  for (int w = 0; w < wave; w++) v = op(s_w[w], v);
-  __syncthreads();
-  return v;
+// 64-position chunks per k_attn_av block: a head's blocks stay within DSH_ATTN_PARTS.
+__device__ __forceinline__ int attn_chunks_per_part(int n) {
+  return ((n + 63) / 64 + DSH_ATTN_PARTS - 1) / DSH_ATTN_PARTS;
 }
 
-// ds_dot_f32 in its AVX-512 order for n % 64 == 0 (ds_kernels_avx.c:357-377): four 16-lane
-// accumulators over 64-element blocks, added pairwise, then the reduce tree. q in LDS, k global.
-__device__ __forceinline__ float attn_dot(const float *q, const float *k, int n) {
-  float a[4][16];
-#pragma unroll
-  for (int m = 0; m < 4; m++)
-#pragma unroll
-    for (int l = 0; l < 16; l++) a[m][l] = 0.0f;
-#pragma unroll
-  for (int i = 0; i < n; i += 64) {
-#pragma unroll
-    for (int m = 0; m < 4; m++) {
-#pragma unroll
-      for (int c = 0; c < 4; c++) {
-        const f32x4 kv = ((const f32x4 *)(k + i + 16 * m))[c];
-        const f32x4 qv = ((const f32x4 *)(q + i + 16 * m))[c];
-#pragma unroll
-        for (int e = 0; e < 4; e++) a[m][4 * c + e] = __builtin_fmaf(qv[e], kv[e], a[m][4 * c + e]);
-      }
-    }
-  }
-  float A16[16];
-#pragma unroll
-  for (int l = 0; l < 16; l++) A16[l] = (a[0][l] + a[1][l]) + (a[2][l] + a[3][l]);
-  float T3[8], T6[4];
-#pragma unroll
-  for (int i = 0; i < 8; i++) T3[i] = A16[8 + i] + A16[i];
-#pragma unroll
-  for (int j = 0; j < 4; j++) T6[j] = T3[4 + j] + T3[j];
-  return (T6[0] + T6[2]) + (T6[1] + T6[3]);
+// A DPP move with the value id in lanes that have no source.
+template <int CTRL>
+__device__ __forceinline__ float attn_dpp_or(float v, float id) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(id), __float_as_int(v), CTRL, 0xF, 0xF, false));
+}
+
+// Scans by DPP within the 16-lane rows (an LDS permute per step of a wave-wide scan costs several times
+// the latency). attn_row_max_incl: running maximum up to the lane; attn_row_mul_incl: product from the lane on.
+__device__ __forceinline__ float attn_row_max_incl(float v) {
+  const float lo = -__builtin_huge_valf();
+  v = fmaxf(v, attn_dpp_or<0x111>(v, lo));  // row_shr:1, 2, 4, 8
+  v = fmaxf(v, attn_dpp_or<0x112>(v, lo));
+  v = fmaxf(v, attn_dpp_or<0x114>(v, lo));
+  return fmaxf(v, attn_dpp_or<0x118>(v, lo));
+}
+__device__ __forceinline__ float attn_row_mul_incl(float v) {
+  v *= attn_dpp_or<0x101>(v, 1.0f);  // row_shl:1, 2, 4, 8
+  v *= attn_dpp_or<0x102>(v, 1.0f);
+  v *= attn_dpp_or<0x104>(v, 1.0f);
+  return v * attn_dpp_or<0x108>(v, 1.0f);
 }
 
 // The attended positions of the token at cache position pos: p < r1 is position p, then r2 + (p - r1)
@@ -221,190 +276,292 @@ __device__ __forceinline__ attn_span attn_positions(int pos, int prefill_len, in
   return sp;
 }
 
-// The optional per-head norms (ds_rms_norm_per_head) and RoPE of one head's q and k (in LDS, hd
-// threads of the block active). Called by every thread of the block.
-__device__ void attn_rope_head(const dsh_attn_t &A, int h, int pos, float *s_q, float *s_k, float *s_r) {
-  const int hd = A.head_dim, half = hd / 2, tid = threadIdx.x;
-  const float *cs = A.rope_cos + (size_t)pos * hd, *sn = A.rope_sin + (size_t)pos * hd;
-  for (int d = tid; d < hd; d += blockDim.x) {
-    s_q[d] = A.q[h * hd + d];
-    s_k[d] = A.k[h * hd + d];
+// The per-head norms (ds_rms_norm_per_head; each optional) and RoPE of one head's q and k (into LDS, one
+// dimension per thread). Called by every thread of a block of at least HD threads.
+template <int HD>
+__device__ void attn_rope_head(const dsh_attn_t &A, int h, int pos, float *s_q, float *s_k) {
+  const int t = threadIdx.x, half = HD / 2;
+  const float *cs = A.rope_cos + (size_t)pos * HD, *sn = A.rope_sin + (size_t)pos * HD;
+  if (t < HD) {
+    s_q[t] = A.q[h * HD + t];
+    s_k[t] = A.k[h * HD + t];
   }
   __syncthreads();
-  for (int which = 0; which < 2; which++) {
-    const float *nw = which ? A.k_norm : A.q_norm;
-    float *v = which ? s_k : s_q;
-    if (nw) {
-      const float r = attn_rms_scale(v, hd, A.eps, s_r);
-      float y[DSH_ATTN_MAX_HD / 64];
-      for (int d = tid, i = 0; d < hd; d += blockDim.x, i++) y[i] = (v[d] * nw[d]) * r;
-      __syncthreads();
-      for (int d = tid, i = 0; d < hd; d += blockDim.x, i++) v[d] = y[i];
-      __syncthreads();
-    }
+  const float rq = A.q_norm ? attn_rms_scale<HD>(s_q, A.eps) : 0.0f;
+  const float rk = A.k_norm ? attn_rms_scale<HD>(s_k, A.eps) : 0.0f;
+  __syncthreads();
+  if (t < HD) {
+    if (A.q_norm) s_q[t] = (s_q[t] * A.q_norm[t]) * rq;
+    if (A.k_norm) s_k[t] = (s_k[t] * A.k_norm[t]) * rk;
   }
-  float rq[DSH_ATTN_MAX_HD / 64], rk[DSH_ATTN_MAX_HD / 64];
-  for (int t = tid, i = 0; t < hd; t += blockDim.x, i++) {
+  __syncthreads();
+  float vq = 0.0f, vk = 0.0f;
+  if (t < HD) {
     const int d = t < half ? t : t - half;
     const float q1 = s_q[d], q2 = s_q[d + half], k1 = s_k[d], k2 = s_k[d + half];
     if (t < half) {
-      rq[i] = __builtin_fmaf(q1, cs[d], -(q2 * sn[d]));
-      rk[i] = __builtin_fmaf(k1, cs[d], -(k2 * sn[d]));
+      vq = __builtin_fmaf(q1, cs[d], -(q2 * sn[d]));
+      vk = __builtin_fmaf(k1, cs[d], -(k2 * sn[d]));
     } else {
-      rq[i] = __builtin_fmaf(q1, sn[t], q2 * cs[t]);
-      rk[i] = __builtin_fmaf(k1, sn[t], k2 * cs[t]);
+      vq = __builtin_fmaf(q1, sn[t], q2 * cs[t]);
+      vk = __builtin_fmaf(k1, sn[t], k2 * cs[t]);
     }
   }
   __syncthreads();
-  for (int t = tid, i = 0; t < hd; t += blockDim.x, i++) {
-    s_q[t] = rq[i];
-    s_k[t] = rk[i];
+  if (t < HD) {
+    s_q[t] = vq;
+    s_k[t] = vk;
   }
   __syncthreads();
 }
 
-// Scores, bit-exact: 64 attended positions per 64-thread block (grid: heads x chunks of the cache),
-// one thread per position; sc[h][p] = ds_dot_f32(q, k_j) * (1/sqrtf(head_dim)). Every block ropes
-// the head's q (and k) itself; the block holding the token's own position writes its roped k into
-// the K cache row pos and uses it from LDS.
-template <int HD>
-__global__ void __launch_bounds__(64) k_attn_scores(dsh_attn_t A, const int *pos_ptr, int pos_add, int prefill_len,
-                                                    int window) {
-  __shared__ __attribute__((aligned(16))) float s_q[HD], s_k[HD];
-  __shared__ float s_r;
-  const int h = blockIdx.x, p = blockIdx.y * 64 + threadIdx.x;
+// Attended positions per score block, and per maximum that a wave of it leaves in A.cm.
+#define ATTN_SCH 64
+#define ATTN_MCH 16
+
+// Scores, bit-exact: 64 attended positions per 256-thread block (grid: heads x chunks of the cache), 16
+// lanes per position, whole cache lines per load and every K row of a wave (16 positions) in flight at once;
+// sc[h][p] = ds_dot_f32(q, k_j) * (1/sqrtf(head_dim)) and cm[h][p/16] the maximum of 16 scores. The order is
+// ds_dot_f32's (ds_kernels_avx.c:357-377, head_dim % 64 == 0): four 16-lane accumulators over 64-column
+// blocks, added pairwise, then the tree. Lane c holds 4 columns of each block; lane quads 0..3 hold accumulators
+// 0, 2, 1, 3, so that lanes c and c ^ 8 hold the first pairs, and after that add the values repeat as the
+// rotation by 4 needs.
+// NORM: the block norms and ropes q and k itself, and the one that holds the token's own position
+// writes its k into the cache row pos. 3.4 us at 702 positions, 7.5 at 7002 (36 MB, 4.8 TB/s); one thread per
+// position (a row of 512 bytes per lane) took 5.7 and 13.5.
+template <int HD, bool NORM>
+__global__ void __launch_bounds__(256) k_attn_scores(dsh_attn_t A, const int *pos_ptr, int pos_add, int prefill_len,
+                                                     int window) {
+  constexpr int NB = HD / 64, PW = ATTN_MCH / 4;
+  __shared__ __attribute__((aligned(16))) float s_q[NORM ? HD : 4], s_k[NORM ? HD : 4];
+  const int h = blockIdx.x, c = threadIdx.x & 15;
+  const int col4 = 8 * ((c >> 2) & 1) + 4 * (c >> 3) + (c & 3);
   const int pos = attn_pos(pos_ptr, pos_add);
   const attn_span sp = attn_positions(pos, prefill_len, window);
-  if ((int)blockIdx.y * 64 >= sp.n) return;  // whole block
-  attn_rope_head(A, h, pos, s_q, s_k, &s_r);
-  const bool own = ((int)blockIdx.y + 1) * 64 >= sp.n;  // this block holds position n-1 == pos
-  if (own)
-    for (int d = threadIdx.x; d < HD; d += 64) A.kc[(size_t)pos * A.kv_stride + h * HD + d] = s_k[d];
-  if (p < sp.n) {
-    const int j = sp.j(p);
-    const float scale = 1.0f / __builtin_sqrtf((float)HD);
-    A.sc[(size_t)h * A.max_seq + p] =
-        attn_dot(s_q, j == pos ? s_k : A.kc + (size_t)j * A.kv_stride + h * HD, HD) * scale;
+  if ((int)blockIdx.y * ATTN_SCH >= sp.n) return;  // whole block
+  const int p0 = blockIdx.y * ATTN_SCH + (threadIdx.x >> 6) * ATTN_MCH + ((threadIdx.x & 63) >> 4);
+  f32x4 kv[PW][NB], q[NB];
+#pragma unroll
+  for (int i = 0; i < PW; i++) {
+    const float *kr = A.kc + (size_t)sp.j(min(p0 + 4 * i, sp.n - 1)) * A.kv_stride + h * HD;
+#pragma unroll
+    for (int b = 0; b < NB; b++) kv[i][b] = ((const f32x4 *)kr)[16 * b + col4];
   }
+  if (NORM) {
+    attn_rope_head<HD>(A, h, pos, s_q, s_k);
+    // this block holds position n-1 == pos
+    if (((int)blockIdx.y + 1) * ATTN_SCH >= sp.n && (int)threadIdx.x < HD)
+      A.kc[(size_t)pos * A.kv_stride + h * HD + threadIdx.x] = s_k[threadIdx.x];
+#pragma unroll
+    for (int i = 0; i < PW; i++)
+      if (p0 + 4 * i >= sp.n - 1)
+#pragma unroll
+        for (int b = 0; b < NB; b++) kv[i][b] = ((const f32x4 *)s_k)[16 * b + col4];
+  }
+#pragma unroll
+  for (int b = 0; b < NB; b++) q[b] = ((const f32x4 *)(NORM ? s_q : A.q + h * HD))[16 * b + col4];
+  const float scale = 1.0f / __builtin_sqrtf((float)HD);
+  float mx = -__builtin_huge_valf();
+#pragma unroll
+  for (int i = 0; i < PW; i++) {
+    float a[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      a[e] = 0.0f;
+#pragma unroll
+      for (int b = 0; b < NB; b++) a[e] = __builtin_fmaf(q[b][e], kv[i][b][e], a[e]);
+      a[e] += dsh_dpp<0x128>(a[e]);  // accumulators 0+1 and 2+3
+      a[e] += dsh_dpp<0x124>(a[e]);  // their sum
+      a[e] += dsh_dpp<0x4E>(a[e]);  // T3: columns 8+i and i are lanes c + 2 and c
+      a[e] += dsh_dpp<0xB1>(a[e]);  // T6
+    }
+    const float s = ((a[0] + a[2]) + (a[1] + a[3])) * scale;
+    if (p0 + 4 * i < sp.n) {
+      if (c == 0) A.sc[(size_t)h * A.max_seq + p0 + 4 * i] = s;
+      mx = fmaxf(mx, s);  // a NaN score is never a new maximum: fmaxf skips it
+    }
+  }
+  mx = fmaxf(mx, __shfl_xor(mx, 16));
+  mx = fmaxf(mx, __shfl_xor(mx, 32));
+  if ((threadIdx.x & 63) == 0) A.cm[(size_t)h * DSH_ATTN_CM(A.max_seq) + p0 / ATTN_MCH] = mx;
 }
 
-// Per head: the reference's sequence of branches (see the top of this file) as coefficients:
-// sc[h][p] <- c_p, se[h] <- sum_e. Dynamic LDS: 2 * max_seq floats.
-__global__ void __launch_bounds__(ATTN_THREADS) k_attn_coef(dsh_attn_t A, const int *pos_ptr, int pos_add,
-                                                            int prefill_len, int window) {
-  extern __shared__ __attribute__((aligned(16))) float s_dyn[];
-  __shared__ float s_w[4];
-  __shared__ __attribute__((aligned(16))) float s_o[ATTN_THREADS];
-  float *s_s = s_dyn, *s_c = s_dyn + A.max_seq;
-  const int h = blockIdx.x, tid = threadIdx.x;
-  const int n = attn_positions(attn_pos(pos_ptr, pos_add), prefill_len, window).n;
-  float *sc = A.sc + (size_t)h * A.max_seq;
-  for (int p = tid; p < n; p += ATTN_THREADS) s_s[p] = sc[p];
-  __syncthreads();
-  // running maximum before each position: exclusive prefix max over contiguous segments
-  const int seg = (n + ATTN_THREADS - 1) / ATTN_THREADS;
-  const int p0 = min(tid * seg, n), p1 = min(p0 + seg, n);
-  float sm = -__builtin_huge_valf();
-  for (int p = p0; p < p1; p++) sm = fmaxf(sm, s_s[p]);
-  const float incl = attn_block_scan(sm, [](float a, float b) { return fmaxf(a, b); }, s_w);
-  s_o[tid] = incl;
-  __syncthreads();
-  // the reference starts from max_s = -1e30 (a NaN score is never a new maximum: fmaxf skips it)
-  float P = fmaxf(-1e30f, tid ? s_o[tid - 1] : -__builtin_huge_valf());
-  __syncthreads();
-  // factors: a = correction on a new maximum (else 1), g = 1 on a new maximum (else the weight);
-  // s_s[p] <- a, s_c[p] <- g
-  float prod = 1.0f;
-  for (int p = p0; p < p1; p++) {
-    const float s = s_s[p];
-    const bool nm = s > P;
-    const float f = dsh_fast_expf(nm ? P - s : s - P);
-    s_s[p] = nm ? f : 1.0f;
-    s_c[p] = nm ? 1.0f : f;
-    prod *= nm ? f : 1.0f;
-    P = nm ? s : P;
-  }
-  // product of the corrections after each segment: a scan over the threads in reverse order
-  // (thread t holds segment ATTN_THREADS-1-t's product; the exclusive suffix of segment tid is the
-  // inclusive value of thread ATTN_THREADS-2-tid)
-  s_o[tid] = prod;
-  __syncthreads();
-  const float rprod = s_o[ATTN_THREADS - 1 - tid];
-  __syncthreads();
-  const float rincl = attn_block_scan(rprod, [](float a, float b) { return a * b; }, s_w);
-  s_o[tid] = rincl;
-  __syncthreads();
-  float after = tid < ATTN_THREADS - 1 ? s_o[ATTN_THREADS - 2 - tid] : 1.0f;
-  float csum = 0.0f;
-  for (int p = p1 - 1; p >= p0; p--) {
-    const float c = s_c[p] * after;  // c = g * (product of the later corrections)
-    sc[p] = c;
-    csum += c;
-    after *= s_s[p];
-  }
-  const float tot = attn_block_scan(csum, [](float a, float b) { return a + b; }, s_w);
-  if (tid == ATTN_THREADS - 1) A.se[h] = tot;
-}
-
-// V: 32 attended positions per block of head_dim threads (grid: heads x chunks), every v load of a
-// thread in flight together; part[h][chunk][d] = sum over the chunk of c_p * v_p[d].
-#define ATTN_VCH 32
-__global__ void __launch_bounds__(DSH_ATTN_MAX_HD) k_attn_av(dsh_attn_t A, const int *pos_ptr, int pos_add,
-                                                             int prefill_len, int window) {
-  __shared__ float s_c[ATTN_VCH];
-  const int h = blockIdx.x, hd = A.head_dim, d = threadIdx.x, p0 = blockIdx.y * ATTN_VCH;
+// V: up to four 64-position chunks per 256-thread block (grid: heads x DSH_ATTN_PARTS), as many as keep a
+// head's blocks within DSH_ATTN_PARTS, so that the next kernel has few sums to put together: one up to 1920
+// positions (160 blocks for 10 heads at 1000), four at 7680. Wave w computes the coefficients of chunk w
+// (lane = position): with P the maximum of the scores before the position (the reference starts from
+// max_s = -1e30), a = its correction on a new maximum (else 1), g = 1 on a new maximum (else the weight),
+// c = g * (the product of the later corrections of the chunk). Then every thread adds c * v for 4 dimensions
+// of 1024/HD-th of the positions, its loads issued before the coefficients are known, and the block writes
+// its sum, its sum of c and its product of corrections. 3.8 us at 702 positions, 8.3 at 7002 (36 MB), against 8.9
+// and 25.7 for a kernel with one block per head for the coefficients and one for the sums.
+template <int HD>
+__global__ void __launch_bounds__(256) k_attn_av(dsh_attn_t A, const int *pos_ptr, int pos_add, int prefill_len,
+                                                 int window) {
+  constexpr int DL = HD / 4, G = 256 / DL, NP = (64 + G - 1) / G;  // lanes per row, rows at once, rows per thread
+  __shared__ float s_c[4][64], s_a[4], s_e[4];
+  __shared__ __attribute__((aligned(16))) float s_o[G * HD];
+  const int h = blockIdx.x, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const attn_span sp = attn_positions(attn_pos(pos_ptr, pos_add), prefill_len, window);
+  const int g = attn_chunks_per_part(sp.n);
+  const int p0 = blockIdx.y * g * 64;
   if (p0 >= sp.n) return;  // whole block
-  const int cnt = min(ATTN_VCH, sp.n - p0);
-  if (d < ATTN_VCH) s_c[d] = d < cnt ? A.sc[(size_t)h * A.max_seq + p0 + d] : 0.0f;
-  float v[ATTN_VCH];
+  const int nc = min(g, (sp.n - p0 + 63) / 64);
+  const int d4 = threadIdx.x % DL, pg = threadIdx.x / DL;  // HD 192: the last 16 threads have pg == G
+  const float *vh = A.vc + h * HD;
+  f32x4 v[NP];
+  auto load = [&](int ch) {
 #pragma unroll
-  for (int q = 0; q < ATTN_VCH; q++) v[q] = A.vc[(size_t)sp.j(p0 + min(q, cnt - 1)) * A.kv_stride + h * hd + d];
-  __syncthreads();
-  float acc = 0.0f;
+    for (int i = 0; i < NP; i++)
+      v[i] = ((const f32x4 *)(vh + (size_t)sp.j(min(p0 + 64 * ch + pg + G * i, sp.n - 1)) * A.kv_stride))[d4];
+  };
+  if (wave < nc) {
+    const int q0 = p0 + 64 * wave, p = q0 + lane;
+    const float *cm = A.cm + (size_t)h * DSH_ATTN_CM(A.max_seq);
+    const int nm = q0 / ATTN_MCH;  // maxima before the chunk
+    float t[DSH_ATTN_CM_MAX / 64];
+    const float sp0 = A.sc[(size_t)h * A.max_seq + min(p, sp.n - 1)];
 #pragma unroll
-  for (int q = 0; q < ATTN_VCH; q++) acc = __builtin_fmaf(s_c[q], v[q], acc);  // s_c is 0 past cnt
-  A.part[((size_t)h * (A.max_seq / ATTN_VCH + 1) + blockIdx.y) * hd + d] = acc;
-}
-
-// Per head: the chunk sums in chunk order, times 1/sum_e (ds_vec_scale_inplace; sum_e > 0).
-__global__ void __launch_bounds__(DSH_ATTN_MAX_HD) k_attn_combine(dsh_attn_t A, const int *pos_ptr, int pos_add,
-                                                                  int prefill_len, int window) {
-  const int h = blockIdx.x, hd = A.head_dim, d = threadIdx.x;
-  const int n = attn_positions(attn_pos(pos_ptr, pos_add), prefill_len, window).n;
-  const int nch = (n + ATTN_VCH - 1) / ATTN_VCH;
-  const float *pt = A.part + (size_t)h * (A.max_seq / ATTN_VCH + 1) * hd + d;
-  float o = 0.0f;
-  for (int c0 = 0; c0 < nch; c0 += 16) {  // 16 loads in flight, then the adds in chunk order
-    float v[16];
+    for (int k = 0; k < DSH_ATTN_CM_MAX / 64; k++) t[k] = cm[min(lane + 64 * k, max(nm - 1, 0))];
+    load(0);
+    __builtin_amdgcn_sched_barrier(0);  // every load is on its way before the first wait
+    const float s = p < sp.n ? sp0 : -__builtin_huge_valf();
+    float before = -1e30f;
 #pragma unroll
-    for (int q = 0; q < 16; q++) v[q] = pt[(size_t)min(c0 + q, nch - 1) * hd];
+    for (int k = 0; k < DSH_ATTN_CM_MAX / 64; k++) before = fmaxf(before, lane + 64 * k < nm ? t[k] : -1e30f);
+    before = dsh_wave_max(before);
+    // maximum of the scores before the lane: the row's, and the rows before it
+    const int row = lane >> 4;
+    const float m = attn_row_max_incl(s);
+    float P = fmaxf(before, attn_dpp_or<0x111>(m, -1e30f));
 #pragma unroll
-    for (int q = 0; q < 16; q++)
-      if (c0 + q < nch) o += v[q];
+    for (int k = 0; k < 3; k++) P = fmaxf(P, row > k ? dsh_readlane(m, 16 * k + 15) : -1e30f);
+    const bool nw = s > P;
+    const float f = dsh_fast_expf(nw ? P - s : s - P);
+    const bool in = p < sp.n;
+    // product of the corrections after the lane: the row's, and the rows after it
+    const float mul = attn_row_mul_incl(in && nw ? f : 1.0f);
+    const float m1 = dsh_readlane(mul, 16), m2 = dsh_readlane(mul, 32), m3 = dsh_readlane(mul, 48);
+    const float rows = row == 0 ? m1 * (m2 * m3) : (row == 1 ? m2 * m3 : (row == 2 ? m3 : 1.0f));
+    const float dn = attn_dpp_or<0x101>(mul, 1.0f) * rows;
+    const float after = dsh_readlane(mul, 0) * (m1 * (m2 * m3));
+    const float cf = in ? (nw ? 1.0f : f) * dn : 0.0f;
+    s_c[wave][lane] = cf;
+    const float se = dsh_wave_sum(cf);
+    if (lane == 0) {
+      s_a[wave] = after;
+      s_e[wave] = se;
+    }
+  } else {
+    load(0);
   }
-  const float se = A.se[h];
-  if (se > 0.0f) o = o * (1.0f / se);
-  A.att[h * hd + d] = o;
+  __syncthreads();
+  f32x4 o = {0.0f, 0.0f, 0.0f, 0.0f};
+  float se = 0.0f, prod = 1.0f;
+  for (int ch = 0; ch < nc; ch++) {
+    const float fall = s_a[ch];
+    o *= fall;  // the chunks before it (nothing yet at the first)
+    se = se * fall + s_e[ch];
+    prod *= fall;
+    f32x4 cur[NP];
+#pragma unroll
+    for (int i = 0; i < NP; i++) cur[i] = v[i];
+    if (ch + 1 < nc) load(ch + 1);
+#pragma unroll
+    for (int i = 0; i < NP; i++) {
+      const int p = pg + G * i;
+      const float cf = p < 64 ? s_c[ch][p] : 0.0f;
+#pragma unroll
+      for (int e = 0; e < 4; e++) o[e] = __builtin_fmaf(cf, cur[i][e], o[e]);
+    }
+  }
+  if (pg < G) ((f32x4 *)s_o)[pg * DL + d4] = o;
+  __syncthreads();
+  const int part = h * DSH_ATTN_PARTS + blockIdx.y;
+  if ((int)threadIdx.x < HD) {
+    float sum = 0.0f;
+#pragma unroll
+    for (int k = 0; k < G; k++) sum += s_o[k * HD + threadIdx.x];
+    A.part[(size_t)part * HD + threadIdx.x] = sum;
+  }
+  if (threadIdx.x == 0) {
+    A.pa[part] = prod;
+    A.pe[part] = se;
+  }
 }
 
 // ---------------------------------------------------------------------------- O projection
-// 16 output rows per 64-thread block; att (q_dim == 32*N32) staged in LDS.
+// 16 output rows per block (threads past 256 only help with att); every block puts att together itself (head h: the parts' sums times
+// the product of the later parts' corrections, in part order, times 1/sum_e: ds_vec_scale_inplace, sum_e > 0),
+// at most 30 x q_dim floats from L2, which costs less than a launch of its own: 5.7 us in all at 702 positions
+// and 6.6 at 7002, against 5.8 + 3.7 and 5.0 + 9.9 in two kernels. q_dim == 32*N32.
 template <int N32>
-__global__ void __launch_bounds__(64) k_attn_oproj(dsh_attn_t A, int chunk) {
-  constexpr int QD = 32 * N32;
+__global__ void __launch_bounds__(attn_threads(32 * N32)) k_attn_oproj(dsh_attn_t A, const int *pos_ptr, int pos_add, int prefill_len,
+                                                    int window, int chunk) {
+  constexpr int QD = 32 * N32, PP = 16;  // parts in flight
   __shared__ __attribute__((aligned(16))) float s_a[QD];
-  const int L = threadIdx.x & 3;
-  const int r = blockIdx.x * 16 + (threadIdx.x >> 2);
-  const int rc = r < A.H ? r : A.H - 1;
-  const uint16_t *w = A.wo + (size_t)rc * QD;
-  const int path = row_path(rc, A.H, chunk, false);
-  u32x4 wv[N32];
-  if (path != DSH_ROW_SINGLE) attn_row_load<N32>(wv, w, L);
-  for (int i = threadIdx.x; i < QD / 4; i += 64) ((f32x4 *)s_a)[i] = ((const f32x4 *)A.att)[i];
+  __shared__ float s_f[QD / 64 * DSH_ATTN_PARTS], s_inv[QD / 64];
+  const int c = threadIdx.x & 15;
+  const int r = blockIdx.x * 16 + ((threadIdx.x >> 4) & 15);
+  const uint16_t *w = A.wo + (size_t)r * QD;
+  const int path = row_path(r, A.H, chunk, false);
+  const int n = attn_positions(attn_pos(pos_ptr, pos_add), prefill_len, window).n;
+  const int g64 = attn_chunks_per_part(n) * 64, np = (n + g64 - 1) / g64;
+  const int dl = A.head_dim / 4;
+  constexpr int NH = (QD / 64 + 7) / 8;  // heads per half wave, at most
+  f32x4 t[PP];
+  const int i0 = min((int)threadIdx.x, QD / 4 - 1), h0 = i0 / dl;  // the thread's f32x4 piece of att
+  const f32x4 *q = (const f32x4 *)A.part + (size_t)h0 * DSH_ATTN_PARTS * dl + (i0 - h0 * dl);
+  // the factors' inputs, half a wave per head
+  const int hw = (threadIdx.x >> 5) & 7, k = threadIdx.x & 31;
+  float pa[NH], pe[NH];
+#pragma unroll
+  for (int i = 0; i < NH; i++) {
+    const int at = min(hw + 8 * i, A.n_heads - 1) * DSH_ATTN_PARTS + min(k, np - 1);
+    pa[i] = A.pa[at];
+    pe[i] = A.pe[at];
+  }
+#pragma unroll
+  for (int j = 0; j < PP; j++) t[j] = q[(size_t)min(j, np - 1) * dl];
+  uint32_t wv[N32];
+  if (threadIdx.x < 256) attn_row_load<N32>(wv, w, c);
+  __builtin_amdgcn_sched_barrier(0);  // every load is on its way before the first wait
+#pragma unroll
+  for (int i = 0; i < NH; i++) {
+    const int h = hw + 8 * i;
+    const float a = k < np ? pa[i] : 1.0f, e = k < np ? pe[i] : 0.0f;
+    const float mul = attn_row_mul_incl(a), upper = __shfl(mul, 16, 32);
+    const float f = attn_dpp_or<0x101>(mul, 1.0f) * (k < 16 ? upper : 1.0f);
+    float tot = dsh_row16_sum(e * f);
+    tot += __shfl_xor(tot, 16);
+    if (h < A.n_heads) {
+      if (k < DSH_ATTN_PARTS) s_f[h * DSH_ATTN_PARTS + k] = f;
+      if (k == 0) s_inv[h] = tot > 0.0f ? 1.0f / tot : 1.0f;
+    }
+  }
   __syncthreads();
-  const float v = attn_row<N32>(w, wv, s_a, L, path);
-  if (L == 0 && r < A.H) A.proj[r] = v;
+  if (threadIdx.x < QD / 4) {
+    f32x4 o = {0.0f, 0.0f, 0.0f, 0.0f};
+    const float *f = s_f + h0 * DSH_ATTN_PARTS;
+#pragma unroll
+    for (int j = 0; j < PP; j++)
+      if (j < np) o += f[j] * t[j];
+    if (np > PP) {  // the rest, again with every load in flight
+#pragma unroll
+      for (int j = PP; j < DSH_ATTN_PARTS; j++) t[j - PP] = q[(size_t)min(j, np - 1) * dl];
+#pragma unroll
+      for (int j = PP; j < DSH_ATTN_PARTS; j++)
+        if (j < np) o += f[j] * t[j - PP];
+    }
+    ((f32x4 *)s_a)[threadIdx.x] = o * s_inv[h0];
+  }
+  __syncthreads();
+  if (threadIdx.x >= 256) return;
+  f32x2 xv[N32];
+  attn_row_x<N32>(xv, s_a, c);
+  __builtin_amdgcn_sched_barrier(0);
+  const float v = attn_row<N32, false>(w, wv, xv, s_a, 1.0f, c, path);
+  if (c == 0) A.proj[r] = v;
 }
 
 // ---------------------------------------------------------------------------- residual RMSNorm
@@ -418,7 +575,7 @@ __global__ void __launch_bounds__(256) k_attn_post(dsh_attn_t A, const float *x_
                                                    const float *__restrict__ WrT, int E, float *__restrict__ partials) {
   constexpr int H = 32 * N32;
   __shared__ __attribute__((aligned(16))) float s_h[H];
-  __shared__ float s_r, s_n[R];
+  __shared__ float s_n[R];
   const float *x = step ? x_in + (size_t)(*step) * stride : x_in;
   const int r0 = blockIdx.x * R;
   float wr[R];
@@ -431,7 +588,7 @@ __global__ void __launch_bounds__(256) k_attn_post(dsh_attn_t A, const float *x_
     ((f32x4 *)s_h)[i] = xv + pv;
   }
   __syncthreads();
-  const float r = attn_rms_scale(s_h, H, A.eps, &s_r);
+  const float r = attn_rms_scale<H>(s_h, A.eps);
   if (threadIdx.x < R) {
     const int i = r0 + threadIdx.x;
     const float nv = (s_h[i] * A.post_norm[i]) * r;
@@ -452,18 +609,18 @@ __global__ void __launch_bounds__(256) k_attn_post(dsh_attn_t A, const float *x_
 
 // ds_rms_norm of the last hidden state before the LM head (ds_moe_decoder.c:1000), AVX-512 order;
 // trunc: ds_bf16_truncate_array after it (:1016-1018, bf16 simulation of model version 3).
-template <int N32>
-__global__ void __launch_bounds__(256) k_final_norm(const float *__restrict__ x, int ncopies,
-                                                    const float *__restrict__ w, float eps, int trunc,
-                                                    float *__restrict__ out, float *__restrict__ x_out) {
+template <int N32, int NC>
+__global__ void __launch_bounds__(attn_threads(32 * N32))
+    k_final_norm(const float *__restrict__ x, const float *__restrict__ w, float eps, int trunc,
+                 float *__restrict__ out, float *__restrict__ x_out) {
   constexpr int H = 32 * N32;
   __shared__ __attribute__((aligned(16))) float s_x[H];
-  __shared__ float s_r;
-  attn_x_pieces(x, H, ncopies, (int)threadIdx.x < H / 4 ? (int)threadIdx.x : -1,
-                (int)threadIdx.x + 256 < H / 4 ? (int)threadIdx.x + 256 : -1, s_x, x_out);
+  attn_x<H, NC, attn_threads(H)> X;
+  X.load(x, nullptr);
+  X.store(s_x, nullptr, x_out);
   __syncthreads();
-  const float r = attn_rms_scale(s_x, H, eps, &s_r);
-  for (int i = threadIdx.x; i < H; i += 256) {
+  const float r = attn_rms_scale<H>(s_x, eps);
+  for (int i = threadIdx.x; i < H; i += blockDim.x) {
     const float v = (s_x[i] * w[i]) * r;
     out[i] = trunc ? dsh_bf16_round_half_up(v) : v;
   }
@@ -474,11 +631,8 @@ extern "C" {
 int dsh_attn_supported(int H, int n_heads, int head_dim) {
   const int qd = n_heads * head_dim;
   return H % 256 == 0 && H / 256 >= 1 && H / 256 <= 8 && head_dim % 64 == 0 && head_dim <= DSH_ATTN_MAX_HD &&
-         head_dim <= ATTN_THREADS && qd % 256 == 0 && qd / 256 >= 1 && qd / 256 <= 8;
+         qd % 256 == 0 && qd / 256 >= 1 && qd / 256 <= 8;
 }
-
-// scores/factors and coefficients; at least 8 floats (the per-part sums reuse the first ones)
-size_t dsh_attn_core_lds(int max_kv) { return (size_t)2 * max_kv * sizeof(float); }
 
 hipError_t dsh_launch_attn(const dsh_attn_t *A, const float *x_in, const int *step, int stride, int ncopies,
                            float *x_plain, const int *pos_ptr, int pos_add, int prefill_len, int window, int nthreads,
@@ -488,11 +642,14 @@ hipError_t dsh_launch_attn(const dsh_attn_t *A, const float *x_in, const int *st
   if ((ncopies != 1 && ncopies != 8) || (ncopies > 1 && (step || !x_plain))) return hipErrorInvalidValue;
   const float *x_post = ncopies > 1 ? x_plain : x_in;  // the residual kernel reads one plain vector
   const int qd = A->n_heads * A->head_dim;
-#define QKV(N)                                                                                     \
-  case N:                                                                                          \
-    k_attn_qkv<8 * N><<<(3 * qd + 63) / 64, 256, 0, s>>>(*A, x_in, step, stride, ncopies,            \
-                                                          ncopies > 1 ? x_plain : nullptr, pos_ptr, \
-                                                          pos_add, nthreads);                      \
+#define QKV(N)                                                                                              \
+  case N:                                                                                                   \
+    if (ncopies > 1)                                                                                        \
+      k_attn_qkv<8 * N, 8><<<3 * qd / 16, 256, 0, s>>>(*A, x_in, step, stride, x_plain, pos_ptr, pos_add,    \
+                                                       nthreads);                                           \
+    else                                                                                                    \
+      k_attn_qkv<8 * N, 1><<<3 * qd / 16, 256, 0, s>>>(*A, x_in, step, stride, nullptr, pos_ptr, pos_add,    \
+                                                       nthreads);                                           \
     break;
   switch (A->H / 256) {
     QKV(1) QKV(2) QKV(3) QKV(4) QKV(5) QKV(6) QKV(7) QKV(8)
@@ -500,31 +657,27 @@ hipError_t dsh_launch_attn(const dsh_attn_t *A, const float *x_in, const int *st
       return hipErrorInvalidValue;
   }
 #undef QKV
-  const dim3 gs(A->n_heads, (A->max_seq + 63) / 64), gv(A->n_heads, (A->max_seq + ATTN_VCH - 1) / ATTN_VCH);
+  const int nch = (A->max_seq + 63) / 64;
+  const dim3 gs(A->n_heads, nch), gv(A->n_heads, nch < DSH_ATTN_PARTS ? nch : DSH_ATTN_PARTS);
+#define CORE(HD)                                                                                        \
+  case HD:                                                                                              \
+    if (A->q_norm || A->k_norm)                                                                         \
+      k_attn_scores<HD, true><<<gs, 256, 0, s>>>(*A, pos_ptr, pos_add, prefill_len, window);            \
+    else                                                                                                \
+      k_attn_scores<HD, false><<<gs, 256, 0, s>>>(*A, pos_ptr, pos_add, prefill_len, window);           \
+    k_attn_av<HD><<<gv, 256, 0, s>>>(*A, pos_ptr, pos_add, prefill_len, window);                        \
+    break;
   switch (A->head_dim) {
-    case 64:
-      k_attn_scores<64><<<gs, 64, 0, s>>>(*A, pos_ptr, pos_add, prefill_len, window);
-      break;
-    case 128:
-      k_attn_scores<128><<<gs, 64, 0, s>>>(*A, pos_ptr, pos_add, prefill_len, window);
-      break;
-    case 192:
-      k_attn_scores<192><<<gs, 64, 0, s>>>(*A, pos_ptr, pos_add, prefill_len, window);
-      break;
-    case 256:
-      k_attn_scores<256><<<gs, 64, 0, s>>>(*A, pos_ptr, pos_add, prefill_len, window);
-      break;
+    CORE(64) CORE(128) CORE(192) CORE(256)
     default:
       return hipErrorInvalidValue;
   }
-  k_attn_coef<<<A->n_heads, ATTN_THREADS, dsh_attn_core_lds(A->max_seq), s>>>(*A, pos_ptr, pos_add, prefill_len,
-                                                                             window);
-  k_attn_av<<<gv, A->head_dim, 0, s>>>(*A, pos_ptr, pos_add, prefill_len, window);
-  k_attn_combine<<<A->n_heads, A->head_dim, 0, s>>>(*A, pos_ptr, pos_add, prefill_len, window);
+#undef CORE
   const int chunk = dsh_chunk_len(A->H, nthreads);
-#define OP(N)                                                             \
-  case N:                                                                 \
-    k_attn_oproj<8 * N><<<(A->H + 15) / 16, 64, 0, s>>>(*A, chunk);       \
+#define OP(N)                                                                                              \
+  case N:                                                                                                  \
+    k_attn_oproj<8 * N><<<A->H / 16, attn_threads(qd), 0, s>>>(*A, pos_ptr, pos_add, prefill_len, window,  \
+                                                               chunk);                                     \
     break;
   switch (qd / 256) {
     OP(1) OP(2) OP(3) OP(4) OP(5) OP(6) OP(7) OP(8)
@@ -557,9 +710,12 @@ hipError_t dsh_launch_attn(const dsh_attn_t *A, const float *x_in, const int *st
 
 hipError_t dsh_launch_final_norm(const float *x, int ncopies, const float *w, int H, float eps, int trunc, float *out,
                                  float *x_out, hipStream_t s) {
-#define FN(N)                                                                         \
-  case N:                                                                             \
-    k_final_norm<8 * N><<<1, 256, 0, s>>>(x, ncopies, w, eps, trunc, out, x_out);     \
+#define FN(N)                                                                           \
+  case N:                                                                               \
+    if (ncopies > 1)                                                                    \
+      k_final_norm<8 * N, 8><<<1, attn_threads(H), 0, s>>>(x, w, eps, trunc, out, x_out);           \
+    else                                                                                \
+      k_final_norm<8 * N, 1><<<1, attn_threads(H), 0, s>>>(x, w, eps, trunc, out, x_out);           \
     break;
   if (H % 256 || (ncopies != 1 && ncopies != 8)) return hipErrorInvalidValue;
   switch (H / 256) {

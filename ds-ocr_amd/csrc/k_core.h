@@ -183,19 +183,22 @@ int dsh_dec_supported(int H, int I, int E, int K, int SI);
 int dsh_dec_partials(int H); /* partial score rows written per layer in CFG mode */
 /* ---- attention half of a decoder layer, one token (k_attn.hip) ---- */
 #define DSH_ATTN_MAX_HD 256
+#define DSH_ATTN_PARTS 30                          /* sums of V rows per head (four 64-position chunks each at 7680) */
+#define DSH_ATTN_CM(max_seq) ((max_seq) / 16 + 4)  /* score maxima per head: one per 16 positions, whole score blocks */
+#define DSH_ATTN_CM_MAX 512                        /* at least DSH_ATTN_CM(7680), a multiple of 64 */
 typedef struct {
   const uint16_t *wq, *wk, *wv, *wo;         /* bf16 [qd][H] x3, [H][qd] (qd = n_heads*head_dim) */
   const float *in_norm, *post_norm;          /* [H] */
   const float *q_norm, *k_norm;              /* [head_dim] or NULL */
   const float *rope_cos, *rope_sin;          /* [max_seq][head_dim] */
   float *kc, *vc;                            /* [max_seq][kv_stride] */
-  float *q, *k, *att, *proj;                 /* scratch: [qd] x3, [H] */
-  float *sc, *part, *se;                     /* [n_heads][max_seq], [n_heads][max_seq/32+1][head_dim], [n_heads] */
+  float *q, *k, *proj;                       /* scratch: [qd] x2, [H] */
+  float *sc, *cm;                            /* scores [n_heads][max_seq] and their maxima [n_heads][DSH_ATTN_CM] */
+  float *part, *pa, *pe;                     /* [n_heads][DSH_ATTN_PARTS][head_dim], [n_heads][DSH_ATTN_PARTS] x2 */
   int H, n_heads, head_dim, kv_stride, max_seq;
   float eps;
 } dsh_attn_t;
 int dsh_attn_supported(int H, int n_heads, int head_dim);
-size_t dsh_attn_core_lds(int max_kv);
 /* h_out = x + Wo·attention(...), n_out = RMSNorm(h_out) for the token at cache position
  * (pos_ptr ? *pos_ptr : 0) + pos_add; x = x_in + (*step)*stride when step != NULL; ncopies > 1:
  * x = Σ of the copies [ncopies][H] at x_in in copy order (step NULL), also written to x_plain ([H]) for the

@@ -47,7 +47,7 @@ ds_hip_attn_t *ds_hip_attn_create(int hidden, int n_heads, int head_dim, int max
   if (!A) return NULL;
   const size_t H = hidden, qd = (size_t)n_heads * head_dim, hd = head_dim;
   const size_t kv_stride = (qd + 15) & ~(size_t)15; /* rows 64-byte aligned, as the reference's cache */
-  size_t off[17], n = 0;
+  size_t off[18], n = 0;
   int k = 0;
 #define REGION(b) (off[k++] = n, n += al256(b))
   REGION(qd * H * 2);                       /* 0 wq */
@@ -62,10 +62,11 @@ ds_hip_attn_t *ds_hip_attn_create(int hidden, int n_heads, int head_dim, int max
   REGION((size_t)max_seq * hd * 4);         /* 9 sin */
   REGION((size_t)max_seq * kv_stride * 4);  /* 10 K cache */
   REGION((size_t)max_seq * kv_stride * 4);  /* 11 V cache */
-  REGION(qd * 4 * 3 + H * 4);               /* 12 scratch: q, k, att, proj */
-  REGION((size_t)n_heads * max_seq * 4);    /* 13 scores, then coefficients */
-  REGION((size_t)n_heads * (max_seq / 32 + 1) * hd * 4); /* 14 per-chunk V sums */
-  REGION((size_t)n_heads * 4);              /* 15 softmax sums */
+  REGION(qd * 4 * 2 + H * 4);               /* 12 scratch: q, k, proj */
+  REGION((size_t)n_heads * max_seq * 4);    /* 13 scores */
+  REGION((size_t)n_heads * DSH_ATTN_CM(max_seq) * 4); /* 14 their maxima */
+  REGION(qd * DSH_ATTN_PARTS * 4);          /* 15 sums of V rows */
+  REGION((size_t)n_heads * DSH_ATTN_PARTS * 4 * 2); /* 16 their products of corrections, sums of coefficients */
 #undef REGION
   hipError_t e = hipMalloc(&A->arena, n);
   if (e != hipSuccess) {
@@ -109,11 +110,12 @@ ds_hip_attn_t *ds_hip_attn_create(int hidden, int n_heads, int head_dim, int max
   d->vc = (float *)(b + off[11]);
   d->q = (float *)(b + off[12]);
   d->k = d->q + qd;
-  d->att = d->k + qd;
-  d->proj = d->att + qd;
+  d->proj = d->k + qd;
   d->sc = (float *)(b + off[13]);
-  d->part = (float *)(b + off[14]);
-  d->se = (float *)(b + off[15]);
+  d->cm = (float *)(b + off[14]);
+  d->part = (float *)(b + off[15]);
+  d->pa = (float *)(b + off[16]);
+  d->pe = d->pa + (size_t)n_heads * DSH_ATTN_PARTS;
   d->H = hidden;
   d->n_heads = n_heads;
   d->head_dim = head_dim;

@@ -234,7 +234,7 @@ int ds_hip_arena_load(const char *path, ds_hip_layer_t **layers, int max_layers,
  * but the attention's output sum is bit-exact with the reference; that sum differs by f32 rounding.
  * No counterpart object in the reference (its layer keeps these in ds_ctx_t). */
 typedef struct ds_hip_attn ds_hip_attn_t;
-#define DS_HIP_ATTN_MAX_SEQ 7680 /* KV positions per layer (the softmax keeps 2 floats per position in LDS) */
+#define DS_HIP_ATTN_MAX_SEQ 7680 /* KV positions per layer (30 partial sums of at most 256 positions per head) */
 /* Weights: bf16 [n_heads*head_dim][hidden] for wq, wk, wv, bf16 [hidden][n_heads*head_dim] for wo;
  * norms f32 [hidden] (q_norm, k_norm: [head_dim] or NULL). Host arrays, uploaded. */
 ds_hip_attn_t *ds_hip_attn_create(int hidden, int n_heads, int head_dim, int max_seq, float rms_eps, float rope_theta,

@@ -46,7 +46,7 @@ def caches(dev, A, n_pos, qd):
     return out
 
 
-def run(dev, B, H, nh, hd, positions, pre, win, T, qk_norm, prefill_kv=0, seed=40):
+def run(dev, B, H, nh, hd, positions, pre, win, T, qk_norm, prefill_kv=0, seed=40, tol=TOL):
     L = dev.load()
     O = B.oracle()
     qd, max_seq = nh * hd, max(positions) + 1
@@ -76,7 +76,7 @@ def run(dev, B, H, nh, hd, positions, pre, win, T, qk_norm, prefill_kv=0, seed=4
             assert np.array_equal(bits(vg[pos]), bits(Vc.reshape(max_seq, stride)[pos, :qd])), pos
             e = max(rel(hd_.to_array(np.float32), h1), rel(nd_.to_array(np.float32), n1))
             worst = max(worst, e)
-            assert e < TOL, (pos, e)
+            assert e < tol, (pos, e)
         return worst
     finally:
         L.ds_set_threads(1)
@@ -96,6 +96,21 @@ def test_attention_block_deepseek_size_rswa(dev, B):
     for pre, win in ((200, 8), (0, 0)):
         worst = run(dev, B, 1280, 10, 128, list(range(200, 220)), pre, win, 1, False, prefill_kv=200, seed=60)
         print(f"attention block 1280/10x128 R-SWA ({pre},{win}): worst rel err {worst:.2e}")
+
+
+@pytest.mark.parametrize("nh,hd", [(4, 64), (2, 128), (4, 192), (1, 256)])
+@pytest.mark.parametrize("qk_norm", [False, True])
+def test_attention_chunk_edges(dev, B, nh, hd, qk_norm):
+    """Positions around the 16-, 64- and 256-position chunks, around the first length at which a block takes two
+    chunks (1921 positions) and at the cache's last position, for every head size, with T = 3 threads (rows on
+    the single-row path). Both sides add up n weighted rows and n weights in f32, with errors of independent sign:
+    about 4 sqrt(n) 2^-24 relative, on top of the bound for short sums."""
+    for first, count in ((14, 4), (62, 4), (254, 4), (1918, 4), (7679, 1)):
+        n = first + count
+        run(dev, B, 256, nh, hd, list(range(first, n)), 0, 0, 3, qk_norm, prefill_kv=first, seed=80 + hd,
+            tol=TOL + 4 * n ** 0.5 * 2.0 ** -24)
+    run(dev, B, 256, nh, hd, list(range(900, 903)), 700, 130, 3, qk_norm, prefill_kv=900, seed=81 + hd,
+        tol=TOL + 4 * 830 ** 0.5 * 2.0 ** -24)
 
 
 def test_attention_rejects_bad_shapes(dev):
