@@ -35,13 +35,13 @@ typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef int i32x16 __attribute__((ext_vector_type(16)));
 
-#define PF_MT 64    // rows of A per work item: one or two MFMA sub-tiles of 32 rows
-#define PF_GU_N 128 // gate_up: intermediate units per block (128 gate + 128 up weight rows)
-#define PF_DN_N 256 // down: output rows per block
-#define PF_NT_MAX 16  // down: 128-column stages per A row (I, SI <= 2048)
+#define PF_MT 64      // A rows per work item
+#define PF_EU 128     // intermediate units that share a limb exponent in a row of h
+#define PF_NT_MAX 16  // such groups per row of h (I, SI <= 2048)
 #define PF_TB 8     // tokens per DECODE-mode scores block
 #define PF_PLAN_LDS 8192  // (token, slot) entries the plan kernel caches in LDS
 #define PF_NQ 8           // work queues of the fused GEMM kernel: one per XCD
+#define PF_UG 8           // items of one expert that share a queue, at most
 #define PF_DN_TILE 0x80000000u  // tile word: down tile flag | item << 8 | n-tile
 
 // Work queues of the fused GEMM kernel (k_pf_moe), built by the plan kernel.
@@ -402,6 +402,8 @@ __global__ void __launch_bounds__(1024) k_pf_plan(const int *__restrict__ idx, i
   __shared__ int cnt[16][64];
   __shared__ int s_nch[64], s_ich[64];
   __shared__ int s_nr;
+  __shared__ int s_ucls[PF_UG + 1][64], s_utot[PF_UG + 1];  // queue units by size: before expert e, in all
+  __shared__ int s_qgu[PF_NQ][PF_UG + 1], s_qdn[PF_NQ][PF_UG + 1];
   __shared__ int run[16][64];
   __shared__ int cache[PF_PLAN_LDS];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -478,42 +480,118 @@ __global__ void __launch_bounds__(1024) k_pf_plan(const int *__restrict__ idx, i
   if (threadIdx.x == 0) *Q.err = 0;
   __syncthreads();
   if (Q.enable) {
-    // Queue units are the work items: the routed items (cost cost_r in 128-column weight stages)
-    // and the shared-expert items (cost_s). Items are ranked by cost, costlier kind first, then
-    // by item number, and dealt to the queues in snake order (rank 16k + j goes to queue j for
-    // j < 8, to queue 15 - j otherwise), so no queue holds more than ceil(items / PF_NQ) of them.
-    // Each queue lists all its gate_up tiles (item by item, n-tiles adjacent: they share the item's
-    // A rows), then its down tiles, in rank order. Ranks and offsets have closed forms.
+    // Queue units are groups of up to PF_UG items of one expert (an expert's nch items in the fewest groups,
+    // their sizes differing by at most one) and the single shared-expert items. A group's tiles run n-tile by n-tile,
+    // its items side by side, on one XCD, so its weight rows come from HBM once and from that XCD's L2 for the other
+    // items; so do the shared items of one queue. Units are ranked by cost (in 128-column weight stages), then by
+    // expert, and dealt to the queues in snake order (rank 16k + j goes to queue j for j < 8, to queue 15 - j
+    // otherwise), so no queue holds more than the mean and the costliest unit. Each queue lists all its gate_up
+    // tiles, then its down tiles, in rank order. Ranks and offsets have closed forms.
     const int ns = (T + PF_MT - 1) / PF_MT, nr = s_nr, nu = nr + ns;
     const int cost_s = Q.ngu_s * Q.nk_gu + Q.ndn * Q.nk_ds, cost_r = Q.ngu_r * Q.nk_gu + Q.ndn * Q.nk_dr;
-    const bool sh_first = cost_s > cost_r;
-    const int s0 = sh_first ? 0 : nr, s1 = s0 + ns;  // rank range of the shared items
+    if (wave < PF_UG) {  // wave v counts the groups of v + 1 items, lane = expert
+      const int nch = s_nch[lane], ug = (nch + PF_UG - 1) / PF_UG, sz = ug ? nch / ug : 0, big = nch - sz * ug;
+      const int c = wave + 1 == sz ? ug - big : (wave + 1 == sz + 1 ? big : 0);
+      int incl = c;
+#pragma unroll
+      for (int d = 1; d < 64; d <<= 1) {
+        const int o = __shfl_up(incl, d);
+        if (lane >= d) incl += o;
+      }
+      s_ucls[wave + 1][lane] = incl - c;
+      if (lane == 63) s_utot[wave + 1] = incl;
+    }
+    __syncthreads();
+    // rank ranges: classes of routed groups by size, large first, the shared items (class 0) where their cost puts them
+    int st[PF_UG + 1], tot[PF_UG + 1];
+    {
+      int at = 0;
+      bool placed = false;
+#pragma unroll
+      for (int z = PF_UG; z >= 1; z--) {
+        if (!placed && cost_s > z * cost_r) {
+          st[0] = at;
+          at += ns;
+          placed = true;
+        }
+        st[z] = at;
+        tot[z] = s_utot[z];
+        at += tot[z];
+      }
+      if (!placed) st[0] = at;
+      tot[0] = ns;
+    }
     // units of queue q among ranks [0, lim)
     auto cnt = [](int q, int lim) {
       const int r = lim & (2 * PF_NQ - 1);
       return 2 * (lim / (2 * PF_NQ)) + (r > q) + (r > 2 * PF_NQ - 1 - q);
     };
-    // gate_up tiles of queue q among ranks [0, lim)
-    auto gtiles = [&](int q, int lim) {
-      const int sh = cnt(q, min(lim, s1)) - cnt(q, min(lim, s0));
-      return sh * Q.ngu_s + (cnt(q, lim) - sh) * Q.ngu_r;
-    };
-    if (threadIdx.x < PF_NQ) {
+    if (threadIdx.x < PF_NQ) {  // each class's first gate_up and down tile in queue q
       const int q = threadIdx.x;
-      Q.count[q] = gtiles(q, nu) + cnt(q, nu) * Q.ndn;
+      int gu = 0, dn = 0;
+      bool placed = false;
+#pragma unroll
+      for (int z = PF_UG; z >= 0; z--) {
+        if (!placed && (z == 0 || cost_s > z * cost_r)) {
+          const int n = cnt(q, st[0] + tot[0]) - cnt(q, st[0]);
+          s_qgu[q][0] = gu;
+          s_qdn[q][0] = dn;
+          gu += n * Q.ngu_s;
+          dn += n * Q.ndn;
+          placed = true;
+        }
+        if (z > 0) {
+          const int n = z * (cnt(q, st[z] + tot[z]) - cnt(q, st[z]));
+          s_qgu[q][z] = gu;
+          s_qdn[q][z] = dn;
+          gu += n * Q.ngu_r;
+          dn += n * Q.ndn;
+        }
+      }
+#pragma unroll
+      for (int z = 0; z <= PF_UG; z++) s_qdn[q][z] += gu;  // the down tiles follow the gate_up tiles
+      Q.count[q] = gu + dn;
       Q.next[q] = 0;
     }
+    __syncthreads();
     for (int u = threadIdx.x; u < nu; u += 1024) {
       Q.gu_done[u] = 0;
-      const bool shared = u >= nr;
-      const int rank = sh_first ? (shared ? u - nr : ns + u) : u;
+      int z = 0, rank, j, m;  // class, rank of the unit, the item's place in it and its items
+      if (u >= nr) {
+        rank = st[0] + u - nr;
+      } else {
+        int e = 0;  // the item's expert: the last whose first item is not past u (experts without items lie on it)
+#pragma unroll
+        for (int d = 32; d; d >>= 1) e += s_ich[min(e + d, 63)] <= u && e + d < 64 ? d : 0;
+        const int nch = s_nch[e], i = u - s_ich[e], ug = (nch + PF_UG - 1) / PF_UG, sz = nch / ug, big = nch - sz * ug;
+        const int nb = big * (sz + 1);  // the expert's larger groups come first
+        z = i < nb ? sz + 1 : sz;
+        const int g = i < nb ? i / (sz + 1) : (i - nb) / sz;
+        j = i < nb ? i - g * (sz + 1) : i - nb - g * sz;
+        int base = st[1];
+#pragma unroll
+        for (int k = 2; k <= PF_UG; k++) base = z == k ? st[k] : base;
+        rank = base + s_ucls[z][e] + g;
+      }
       const int pos = rank & (2 * PF_NQ - 1);
       const int q = pos < PF_NQ ? pos : 2 * PF_NQ - 1 - pos;
-      const int gu0 = gtiles(q, rank), dn0 = gtiles(q, nu) + cnt(q, rank) * Q.ndn;
+      int base = st[0];
+#pragma unroll
+      for (int k = 1; k <= PF_UG; k++) base = z == k ? st[k] : base;
+      const int before = cnt(q, rank) - cnt(q, base);  // units of the class before it in the queue
       int *qt = Q.tiles + (size_t)q * Q.cap;
-      const int ngu = shared ? Q.ngu_s : Q.ngu_r;
-      for (int nt = 0; nt < ngu; nt++) qt[gu0 + nt] = (u << 8) | nt;
-      for (int nt = 0; nt < Q.ndn; nt++) qt[dn0 + nt] = (int)(PF_DN_TILE | (u << 8) | nt);
+      int gu0 = s_qgu[q][z], dn0 = s_qdn[q][z], ngu = Q.ngu_s;
+      if (z == 0) {  // the queue's shared items are one group
+        j = before;
+        m = cnt(q, st[0] + tot[0]) - cnt(q, st[0]);
+      } else {
+        ngu = Q.ngu_r;
+        m = z;
+        gu0 += before * z * ngu;
+        dn0 += before * z * Q.ndn;
+      }
+      for (int nt = 0; nt < ngu; nt++) qt[gu0 + nt * m + j] = (u << 8) | nt;
+      for (int nt = 0; nt < Q.ndn; nt++) qt[dn0 + nt * m + j] = (int)(PF_DN_TILE | (u << 8) | nt);
     }
   }
   // the pair positions (no barrier: they read only run and the cached entries, both complete)
@@ -566,7 +644,7 @@ __device__ __forceinline__ bool pf_tile(const int *counts, const int *tiles, int
   return true;
 }
 
-// One block computes C[MB·16 A rows][4 waves x 64 weight rows] = A · B^T over K columns on the
+// One block (4 waves) computes C[MB·16 A rows][4 waves x NB·16 weight rows] = A · B^T over K columns on the
 // int8 MFMA (v_mfma_i32_16x16x64_i8): A = activations as two int8 limbs, B = the weights' stored
 // codes. K runs in stages of PF_KS = 128 columns (one 128-byte line of each weight row), two
 // 64-column MFMA slices each; pf_mainloop_i8 below gives the details.
@@ -575,20 +653,29 @@ __device__ __forceinline__ bool pf_tile(const int *counts, const int *tiles, int
 #define PF_OCC 2  // GEMM blocks per CU the register budget is sized for
 #endif
 
+// Tile shape: up to MT A rows, NB 16-row n-blocks per wave. GU intermediate units (their gate and up rows) per
+// gate_up tile, DN output rows per down tile.
+template <int MT_, int NB_>
+struct pf_shape {
+  static constexpr int MT = MT_, NB = NB_, GU = 32 * NB_, DN = 64 * NB_;
+};
+typedef pf_shape<PF_MT, 4> pf_tile_t;
+
+template <typename C>
 struct pf_smem {
   union {
     struct {
-      int8_t A[2][2][PF_MT][PF_KS];  // [stage parity][low, high limb][row][column, swizzled]
+      int8_t A[2][2][C::MT][PF_KS];  // [stage parity][low, high limb][row][column, swizzled]
     } q;                             // main loop
-    float red[4][64][33];  // gate_up epilogue: h values per wave for the row sums
+    float red[4][C::MT][8 * C::NB + 1];  // gate_up epilogue: h values per wave
   } u;
-  float hsum[4][2][32];  // Σh of the block's A rows (per wave, per 32-row half)
-  float hmx[4][2][32];   // gate_up: max |h| of the block's A rows (per wave, per 32-row half)
-  float xs[PF_MT];       // gate_up: Σx of the block's A rows (their tokens)
-  float xsc[PF_MT];      // the A rows' limb scale 2^(e-15)
-  short ek[PF_MT][PF_NT_MAX];  // down: exponent of each A row's n-tiles
-  float hp[PF_MT][PF_NT_MAX];  // down: Σh of each A row's n-tiles (the gate_up partials)
-  int erow[PF_MT];             // down: the A rows' common exponent (max over their n-tiles)
+  float hsum[4][C::MT];  // Σh of the block's A rows (gate_up: per wave)
+  float hmx[4][C::MT];   // gate_up: max |h| of the block's A rows, per wave
+  float xs[C::MT];       // gate_up: Σx of the block's A rows (their tokens)
+  float xsc[C::MT];      // the A rows' limb scale 2^(e-15)
+  short ek[C::MT][PF_NT_MAX];  // down: exponent of each A row's unit groups
+  float hp[C::MT][PF_NT_MAX];  // down: Σh of each A row's unit groups (the gate_up partials)
+  int erow[C::MT];             // down: the A rows' common exponent (max over their groups)
 };
 
 // Limb exponent of a set of values with max |v| = mx: 2^e > mx·(1 + 2^-7), so rint(v·2^(15-e)) + 128
@@ -698,129 +785,164 @@ hipError_t dsh_launch_pf_swiglu_check(unsigned long long *counts, hipStream_t s)
 // distinct bank groups, and two consecutive rows fill 256 contiguous bytes
 __device__ __forceinline__ int pf_swz(int r) { return (r ^ (r >> 3)) & 7; }
 
+// Stages of loads in flight per wave: A and B registers of a stage are reloaded with the stage D later once they
+// are used. A wave's loads return in issue order, so A runs as far ahead as B: an A stage loaded one
+// stage ahead would wait for every weight load issued before it.
+constexpr int pf_depth(int MB) { return MB == 1 ? 3 : (MB == 2 ? 2 : 1); }
+
 // The int8 main loop (both projections). Per 128-column stage:
 // - weights go from HBM straight into the MFMA's B operand registers: for n-block j (16 weight
-//   rows: j = 0, 1 from brow0, 2, 3 from brow1) and slice s, lane l loads bytes 64s + 16(l/16) .. +15
-//   of the stage in row 16j + l%16 (each load instruction reads 16 rows x 64 contiguous bytes); a
-//   slice's registers are reloaded with the next stage's slice as soon as its MFMAs are issued;
-// - A: the block's rows are copied (8 adjacent lanes per row's 128 bytes, one stage ahead in
-//   registers) into a double-buffered LDS tile with 128-byte rows whose 16-byte chunks are
-//   XOR-swizzled by pf_swz(row); lane l reads chunk 4s + l/16 of row 16mb + l%16, the same columns
-//   as its weight bytes, so each MFMA adds the exact products over the slice (A and B share the
-//   order of k inside the instruction, which leaves the sum unchanged);
+//   rows: the first NB/2 from brow0, the others from brow1) and slice s, lane l loads bytes 64s + 16(l/16) .. +15
+//   of the stage in row 16j + l%16 (each load instruction reads 16 rows x 64 contiguous bytes; the two slices' loads
+//   are issued together, so the second finds its lines on their way);
+// - A: the block's rows are copied (8 adjacent lanes per row's 128 bytes) into a double-buffered LDS tile with
+//   128-byte rows whose 16-byte chunks are XOR-swizzled by pf_swz(row); lane l reads chunk 4s + l/16 of
+//   row 16mb + l%16, the same columns as its weight bytes, so each MFMA adds the exact products over the
+//   slice (A and B share the order of k inside the instruction, which leaves the sum unchanged);
 // - one barrier per stage.
 // acc[mb][j][l]: A rows 16mb .. +15, n-block j, limb l (low, high), exact int32 sums; lane l,
 // register i holds A row 16mb + 4(l/16) + i, weight row 16j + l%16. A rows past the item's count
 // repeat a valid row; their results are never stored.
 // A is two int8 limb arrays, A0 low and A1 high (gate_up: x at one exponent per row; down: h at
-// one exponent per row and 128-column stage). ALIGN (down): before a stage's A values go to LDS,
-// each is brought to its row's common exponent (pf_align16 with d = erow - ek of the row's stage;
-// sm.ek, sm.erow; trow: the table rows of this thread's two A rows).
-// pre() runs once the first stage's loads are issued (down: building the alignment table), so its
+// one exponent per row and 64-column half stage). ALIGN (down): before a stage's A values go to LDS,
+// each is brought to its row's common exponent (pf_align16 with d = erow - ek of the row's half stage;
+// sm.ek, sm.erow; trow: the table rows of this thread's A rows).
+// pre() runs once the first stages' loads are issued (down: building the alignment table), so its
 // waits leave them in flight.
-template <int MB, bool ALIGN, typename Pre>
+template <int MB>
+struct pf_arows {  // A rows a thread copies: pf_arow(c), c < N (MB 1: two threads copy the same row's chunk)
+  static constexpr int N = MB == 1 ? 1 : MB / 2;
+  static __device__ __forceinline__ int row(int c) {
+    return MB == 1 ? (int)(threadIdx.x & 127) >> 3 : (int)(threadIdx.x >> 3) + 32 * c;
+  }
+};
+
+template <typename C, int MB, bool ALIGN, typename Pre>
 __device__ __forceinline__ void pf_mainloop_i8(const int8_t *A0, const int8_t *A1, const size_t *arow,
                                                const int *trow, int K, const int8_t *brow0, const int8_t *brow1,
-                                               i32x4 (&acc)[MB][4][2], pf_smem &sm, Pre &&pre) {
+                                               i32x4 (&acc)[MB][C::NB][2], pf_smem<C> &sm, Pre &&pre) {
+  constexpr int NB = C::NB, D = pf_depth(MB), NA = pf_arows<MB>::N;
   const int lane = threadIdx.x & 63, r16 = lane & 15, kg = lane >> 4;
-  const int ar = threadIdx.x >> 3, ac = threadIdx.x & 7;  // A copy: rows ar and ar + 32, chunk ac
+  const int ac = threadIdx.x & 7;  // A copy: chunk ac of the thread's rows
   const int nk = K / PF_KS;
+  const size_t K16 = (size_t)16 * K;
+  const int8_t *p0 = brow0 + (size_t)r16 * K + 16 * kg;
+  const int8_t *p1 = brow1 + (size_t)r16 * K + 16 * kg;
+  i32x4 bR[D][2][NB];    // [stage % D][slice][n-block]
+  u32x4 aR[D][2][NA];    // [stage % D][limb][row]
+  auto load_b = [&](int d, int j, int k) {
+#pragma unroll
+    for (int sl = 0; sl < 2; sl++)
+      bR[d][sl][j] = *(const i32x4 *)((j < NB / 2 ? p0 : p1) + (j % (NB / 2)) * K16 + (size_t)k * PF_KS + 64 * sl);
+    asm volatile("" ::: "memory");
+  };
+  auto load_a = [&](int d, int k) {
+    const size_t o = (size_t)k * PF_KS + 16 * ac;
+#pragma unroll
+    for (int c = 0; c < NA; c++) {
+      aR[d][0][c] = *(const u32x4 *)(A0 + arow[c] + o);
+      aR[d][1][c] = *(const u32x4 *)(A1 + arow[c] + o);
+    }
+    asm volatile("" ::: "memory");
+  };
+  auto store_a = [&](int d, int a, int k) {
+#pragma unroll
+    for (int c = 0; c < NA; c++) {
+      const int r = pf_arows<MB>::row(c), w = 16 * (ac ^ pf_swz(r));
+      if (ALIGN) {
+        const int sh = min(sm.erow[trow[c]] - (int)sm.ek[trow[c]][k], 31);
+        if (sh > 0) pf_align16(aR[d][0][c], aR[d][1][c], sh);
+      }
+      *(u32x4 *)&sm.u.q.A[a][0][r][w] = aR[d][0][c];
+      *(u32x4 *)&sm.u.q.A[a][1][r][w] = aR[d][1][c];
+    }
+  };
+#pragma unroll
+  for (int d = 0; d < D; d++) {
+    load_a(d, min(d, nk - 1));
+#pragma unroll
+    for (int j = 0; j < NB; j++) load_b(d, j, min(d, nk - 1));
+  }
+  pre();
 #pragma unroll
   for (int mb = 0; mb < MB; mb++)
 #pragma unroll
-    for (int j = 0; j < 4; j++)
+    for (int j = 0; j < NB; j++)
 #pragma unroll
       for (int l = 0; l < 2; l++) acc[mb][j][l] = i32x4{0, 0, 0, 0};
-  int zero = 0;
-  asm volatile("" : "+v"(zero) : "v"((int)arow[0]), "v"((int)arow[1]));
-  const size_t K16 = (size_t)16 * K;
-  const int8_t *p0 = brow0 + zero + (size_t)r16 * K + 16 * kg;
-  const int8_t *p1 = brow1 + zero + (size_t)r16 * K + 16 * kg;
-  const int aw0 = 16 * (ac ^ pf_swz(ar)), aw1 = 16 * (ac ^ pf_swz(ar + 32));
-  i32x4 bR[2][4];  // [slice][n-block] of the stage
-  u32x4 aR[4];     // X0 rows ar, ar+32, X1 rows ar, ar+32
-  auto load_b = [&](int sl, int k) {
-#pragma unroll
-    for (int j = 0; j < 4; j++)
-      bR[sl][j] = *(const i32x4 *)((j < 2 ? p0 : p1) + (j & 1) * K16 + (size_t)k * PF_KS + 64 * sl);
-  };
-  auto load_a = [&](int k) {
-    const size_t o = (size_t)k * PF_KS + 16 * ac;
-    aR[0] = *(const u32x4 *)(A0 + arow[0] + o);
-    aR[1] = *(const u32x4 *)(A0 + arow[1] + o);
-    aR[2] = *(const u32x4 *)(A1 + arow[0] + o);
-    aR[3] = *(const u32x4 *)(A1 + arow[1] + o);
-  };
-  auto store_a = [&](int a, int k) {
-    if (ALIGN) {
-#pragma unroll
-      for (int c = 0; c < 2; c++) {
-        const int d = min(sm.erow[trow[c]] - (int)sm.ek[trow[c]][k], 31);
-        if (d > 0) pf_align16(aR[c], aR[2 + c], d);
-      }
-    }
-    *(u32x4 *)&sm.u.q.A[a][0][ar][aw0] = aR[0];
-    *(u32x4 *)&sm.u.q.A[a][0][ar + 32][aw1] = aR[1];
-    *(u32x4 *)&sm.u.q.A[a][1][ar][aw0] = aR[2];
-    *(u32x4 *)&sm.u.q.A[a][1][ar + 32][aw1] = aR[3];
-  };
-  // the same issue order as in the loop (A, then slice 0, then slice 1), so the wait counts the
-  // compiler derives at the loop head leave the weight loads in flight
-  load_a(0);
-  asm volatile("" ::: "memory");
-  load_b(0, 0);
-  asm volatile("" ::: "memory");
-  load_b(1, 0);
-  asm volatile("" ::: "memory");
-  pre();
-#pragma unroll 1
-  for (int k = 0; k < nk; k++) {
-    const int a = k & 1, kn = min(k + 1, nk - 1);
-    store_a(a, k);
-    load_a(kn);
-    asm volatile("" ::: "memory");
+  // stage k, in registers d; LOAD: then reloaded with stage k + D
+  auto stage = [&](int d, int k, bool LOAD) {
+    const int a = k & 1, kn = k + D;
+    store_a(d, a, k);
+    if (LOAD) load_a(d, kn);
     __syncthreads();
+    constexpr int MH = MB < 2 ? MB : 2;  // m-blocks whose A operands are held at once
 #pragma unroll
-    for (int sl = 0; sl < 2; sl++) {
-      i32x4 x0[MB], x1[MB];
+    for (int m0 = 0; m0 < MB; m0 += MH) {
+      i32x4 x[2][MH][2];
 #pragma unroll
-      for (int mb = 0; mb < MB; mb++) {
-        const int m = 16 * mb + r16, c = 16 * ((4 * sl + kg) ^ pf_swz(m));
-        x0[mb] = *(const i32x4 *)&sm.u.q.A[a][0][m][c];
-        x1[mb] = *(const i32x4 *)&sm.u.q.A[a][1][m][c];
-      }
+      for (int sl = 0; sl < 2; sl++)
 #pragma unroll
-      for (int mb = 0; mb < MB; mb++)
+        for (int mb = 0; mb < MH; mb++) {
+          const int m = 16 * (m0 + mb) + r16, c = 16 * ((4 * sl + kg) ^ pf_swz(m));
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-          acc[mb][j][0] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x0[mb], bR[sl][j], acc[mb][j][0], 0, 0, 0);
-          acc[mb][j][1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x1[mb], bR[sl][j], acc[mb][j][1], 0, 0, 0);
+          for (int l = 0; l < 2; l++) x[sl][mb][l] = *(const i32x4 *)&sm.u.q.A[a][l][m][c];
         }
-      load_b(sl, kn);
-      asm volatile("" ::: "memory");
+#pragma unroll
+      for (int j = 0; j < NB; j++) {
+#pragma unroll
+        for (int sl = 0; sl < 2; sl++)
+#pragma unroll
+          for (int mb = 0; mb < MH; mb++)
+#pragma unroll
+            for (int l = 0; l < 2; l++)
+              acc[m0 + mb][j][l] =
+                  __builtin_amdgcn_mfma_i32_16x16x64_i8(x[sl][mb][l], bR[d][sl][j], acc[m0 + mb][j][l], 0, 0, 0);
+        if (LOAD && m0 + MH >= MB) load_b(d, j, kn);
+      }
     }
+  };
+  // whole rounds of D stages that all load another one, then the rest in straight-line code: with an early exit inside
+  // the loop the compiler takes a stage's loads to be the latest ones at the loop's head, and waits for nearly all
+  int k = 0;
+#pragma unroll 1
+  for (; k + 2 * D <= nk; k += D) {
+#pragma unroll
+    for (int d = 0; d < D; d++) stage(d, k + d, true);
   }
+#pragma unroll
+  for (int d = 0; d < 2 * D - 1; d++)
+    if (k + d < nk) stage(d % D, k + d, d < D - 1 && k + d + D < nk);
 }
 
-// gate_up: block = (work item, n-tile): the item's A rows (tokens) x 128 intermediate units; wave w
-// owns units i0 + 32w .. +31: n-blocks 0, 1 = their gate rows, 2, 3 = their up rows, so each SwiGLU
-// pair sits in the same lane and register (n-blocks h and 2 + h).
-template <bool SHARED, int MB>
+__device__ __forceinline__ float pf_row16_max(float v) {  // over each aligned group of 16 lanes
+  v = fmaxf(v, dsh_dpp<0xB1>(v));
+  v = fmaxf(v, dsh_dpp<0x4E>(v));
+  v = fmaxf(v, dsh_dpp<0x141>(v));
+  return fmaxf(v, dsh_dpp<0x140>(v));
+}
+
+// gate_up: block = (work item, n-tile): the item's A rows (tokens) x GU intermediate units; wave w
+// owns the 16·NB/2 units from i0 + 16·NB/2·w: its first NB/2 n-blocks are their gate rows, the others their up rows,
+// so each SwiGLU pair sits in the same lane and register (n-blocks h and NB/2 + h).
+template <typename C, bool SHARED, int MB>
 __device__ __forceinline__ void gate_up_tile(const dsh_layer_t &L, const pf_item &it, int nt, const int8_t *X0,
                                              const int8_t *X1, const float *xsc, const float *xsum,
                                              const int *pair_tok, int bf16sim, int8_t *Hq0, int8_t *Hq1,
-                                             float *hpart, float *hmaxp, pf_smem &sm) {
+                                             float *hpart, float *hmaxp, pf_smem<C> &sm) {
+  constexpr int HB = C::NB / 2, WU = 16 * HB, WG = PF_EU / WU;  // 16-unit blocks and units per wave, waves per group
   const int H = L.H;
-  const int Iseg = SHARED ? L.SI : L.I, ntK = Iseg / PF_GU_N;
+  const int Iseg = SHARED ? L.SI : L.I, ntK = Iseg / PF_EU;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r16 = lane & 15, kg = lane >> 4;
-  const int u0 = nt * PF_GU_N + wave * 32;
+  const int u0 = nt * C::GU + wave * WU;
   const int8_t *wq = SHARED ? L.sgu_q : L.gu_q + (size_t)it.seg * 2 * L.I * H;
   const float *wso = SHARED ? L.sgu_so : L.gu_so + (size_t)it.seg * 2 * L.I * 2;
-  size_t arow[2];
-  int tok[2];
+  constexpr int NA = pf_arows<MB>::N;
+  size_t arow[NA];
+  int tok[NA];
 #pragma unroll
-  for (int c = 0; c < 2; c++) {
-    const int r = (threadIdx.x >> 3) + 32 * c;
+  for (int c = 0; c < NA; c++) {
+    const int r = pf_arows<MB>::row(c);
     const int rr = r < it.mcnt ? r : 0;
     tok[c] = SHARED ? it.m0 + rr : pair_tok[it.pos0 + it.m0 + rr];
     arow[c] = (size_t)tok[c] * H;
@@ -828,36 +950,36 @@ __device__ __forceinline__ void gate_up_tile(const dsh_layer_t &L, const pf_item
   // the rows' Σx and limb scales for the epilogue, staged in LDS (visible after the main loop's
   // first barrier)
   if ((threadIdx.x & 7) == 0) {
-    const float x0 = xsum[tok[0]], x1 = xsum[tok[1]], c0 = xsc[tok[0]], c1 = xsc[tok[1]];
-    sm.xs[threadIdx.x >> 3] = x0;
-    sm.xs[(threadIdx.x >> 3) + 32] = x1;
-    sm.xsc[threadIdx.x >> 3] = c0;
-    sm.xsc[(threadIdx.x >> 3) + 32] = c1;
+#pragma unroll
+    for (int c = 0; c < NA; c++) {
+      const int r = pf_arows<MB>::row(c);
+      sm.xs[r] = xsum[tok[c]];
+      sm.xsc[r] = xsc[tok[c]];
+    }
   }
   // the lane's units' scales and offsets (units u0 + 16h + l%16), loaded before the main loop so
   // the epilogue does not wait for them
-  float2 sog[2], sou[2];
+  float2 sog[HB], sou[HB];
 #pragma unroll
-  for (int h = 0; h < 2; h++) {
+  for (int h = 0; h < HB; h++) {
     const int unit = u0 + 16 * h + r16;
     sog[h] = ((const float2 *)wso)[unit];
     sou[h] = ((const float2 *)wso)[Iseg + unit];
   }
-  i32x4 acc[MB][4][2];
-  pf_mainloop_i8<MB, false>(X0, X1, arow, nullptr, H, wq + (size_t)u0 * H, wq + (size_t)(Iseg + u0) * H, acc, sm,
-                            [] {});
+  i32x4 acc[MB][C::NB][2];
+  pf_mainloop_i8<C, MB, false>(X0, X1, arow, nullptr, H, wq + (size_t)u0 * H, wq + (size_t)(Iseg + u0) * H, acc, sm,
+                               [] {});
   // signed codes: offset + 128·scale multiplies Σa
 #pragma unroll
-  for (int h = 0; h < 2; h++) {
+  for (int h = 0; h < HB; h++) {
     sog[h].y = __builtin_fmaf(128.0f, sog[h].x, sog[h].y);
     sou[h].y = __builtin_fmaf(128.0f, sou[h].x, sou[h].y);
   }
   const size_t rbase = SHARED ? (size_t)it.m0 : (size_t)(it.pos0 + it.m0);
-  // The tile's h values go to LDS (per wave: 64 rows x its 32 units); each lane sums a row (Σh over
-  // the block's 128 units, for the down epilogue's offset term) and takes its max |h|; the rows'
-  // maxima over the block's 128 units give each row's limb exponent for this n-tile, from which the
-  // lanes store 8-unit runs of both limbs.
-  float(*red)[64][33] = sm.u.red;
+  // The tile's h values go to LDS (per wave: its rows x its units); the sums and maxima over a row's units run
+  // by DPP over the 16 lanes that hold them, then over the waves of a group of PF_EU units, whose maximum gives
+  // the group's limb exponent; the lanes then store 8-unit runs of both limbs.
+  float(*red)[C::MT][8 * C::NB + 1] = sm.u.red;
   __syncthreads();  // every wave is done with the main loop's tiles
   // rows past the item's count repeat row 0 (valid values, never stored); the bf16 simulation is
   // one branch around the loop
@@ -865,14 +987,15 @@ __device__ __forceinline__ void gate_up_tile(const dsh_layer_t &L, const pf_item
 #pragma unroll
     for (int mb = 0; mb < MB; mb++)
 #pragma unroll
-      for (int h = 0; h < 2; h++)
+      for (int i = 0; i < 4; i++) {
+        const int m = 16 * mb + 4 * kg + i;
+        const float xs = sm.xs[m], sc = sm.xsc[m];
+        float sum = 0.0f, mx = 0.0f;
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-          const int m = 16 * mb + 4 * kg + i;
-          const float xs = sm.xs[m], sc = sm.xsc[m];
+        for (int h = 0; h < HB; h++) {
           // Σ q·x = 2^(e-15)·(256·Σ q·X1 + Σ q·X0)
           const float dg = sc * __builtin_fmaf(256.0f, (float)acc[mb][h][1][i], (float)acc[mb][h][0][i]);
-          const float du = sc * __builtin_fmaf(256.0f, (float)acc[mb][2 + h][1][i], (float)acc[mb][2 + h][0][i]);
+          const float du = sc * __builtin_fmaf(256.0f, (float)acc[mb][HB + h][1][i], (float)acc[mb][HB + h][0][i]);
           float g = __builtin_fmaf(sog[h].x, dg, sog[h].y * xs);
           float up = __builtin_fmaf(sou[h].x, du, sou[h].y * xs);
           if (decltype(sim)::value) {
@@ -882,36 +1005,36 @@ __device__ __forceinline__ void gate_up_tile(const dsh_layer_t &L, const pf_item
           float hv = pf_swiglu(g, up);
           if (decltype(sim)::value) hv = dsh_bf16_round_half_up(hv);
           red[wave][m][16 * h + r16] = hv;
+          sum += hv;
+          mx = fmaxf(mx, fabsf(hv));
         }
+        sum = dsh_row16_sum(sum);
+        mx = pf_row16_max(mx);
+        if (r16 == 0) {
+          sm.hsum[wave][m] = sum;
+          sm.hmx[wave][m] = mx;
+        }
+      }
   };
   if (bf16sim)
     h_out(std::true_type{});
   else
     h_out(std::false_type{});
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  float part = 0.0f, pmax = 0.0f;  // lane = row: its sum (in unit order) and max |h| over the wave's 32 units
-  if (lane < 16 * MB) {
-#pragma unroll 8
-    for (int u = 0; u < 32; u++) {
-      const float hv = red[wave][lane][u];
-      part += hv;
-      pmax = fmaxf(pmax, fabsf(hv));
-    }
-  }
-  sm.hsum[wave][lane >> 5][lane & 31] = part;
-  sm.hmx[wave][lane >> 5][lane & 31] = pmax;
   __syncthreads();
-  {  // stores: lane → rows (lane / 4) + 16k, units 8·(lane % 4) .. +7 of the wave's 32, as limbs
-    const int g8 = 8 * (lane & 3);
+  auto group_max = [&](int g, int m) {
+    float mx = sm.hmx[g * WG][m];
 #pragma unroll
-    for (int k = 0; k < MB; k++) {
-      const int m = (lane >> 2) + 16 * k;
+    for (int w = 1; w < WG; w++) mx = fmaxf(mx, sm.hmx[g * WG + w][m]);
+    return mx;
+  };
+  {  // stores: lane → row lane / LR + (64 / LR)·k, units 8·(lane % LR) .. +7 of the wave's, as limbs
+    constexpr int LR = WU / 8, RP = 64 / LR;
+    const int g8 = 8 * (lane % LR);
+#pragma unroll
+    for (int k = 0; k < (16 * MB + RP - 1) / RP; k++) {
+      const int m = lane / LR + RP * k;
       if (m >= it.mcnt) continue;
-      const int a = m >> 5, b = m & 31;
-      const float mx = fmaxf(fmaxf(sm.hmx[0][a][b], sm.hmx[1][a][b]), fmaxf(sm.hmx[2][a][b], sm.hmx[3][a][b]));
-      const float f = __builtin_ldexpf(1.0f, 15 - pf_limb_exp(mx));
+      const float f = __builtin_ldexpf(1.0f, 15 - pf_limb_exp(group_max(wave / WG, m)));
       f32x4 v0, v1;
 #pragma unroll
       for (int i = 0; i < 4; i++) {
@@ -927,23 +1050,29 @@ __device__ __forceinline__ void gate_up_tile(const dsh_layer_t &L, const pf_item
     }
   }
   if (threadIdx.x < it.mcnt) {
-    const int m = threadIdx.x, a = m >> 5, b = m & 31;
-    const float tot = ((sm.hsum[0][a][b] + sm.hsum[1][a][b]) + sm.hsum[2][a][b]) + sm.hsum[3][a][b];
-    const float mx = fmaxf(fmaxf(sm.hmx[0][a][b], sm.hmx[1][a][b]), fmaxf(sm.hmx[2][a][b], sm.hmx[3][a][b]));
-    hpart[(rbase + m) * ntK + nt] = tot;
-    hmaxp[(rbase + m) * ntK + nt] = mx;
+    const int m = threadIdx.x;
+#pragma unroll
+    for (int g = 0; g < C::GU / PF_EU; g++) {
+      float tot = sm.hsum[g * WG][m];
+#pragma unroll
+      for (int w = 1; w < WG; w++) tot += sm.hsum[g * WG + w][m];
+      hpart[(rbase + m) * ntK + nt * (C::GU / PF_EU) + g] = tot;
+      hmaxp[(rbase + m) * ntK + nt * (C::GU / PF_EU) + g] = group_max(g, m);
+    }
   }
 }
 
-template <bool SHARED>
+template <typename C, bool SHARED>
 __device__ __forceinline__ void gate_up_dispatch(const dsh_layer_t &L, const pf_item &it, int nt, const int8_t *X0,
                                                  const int8_t *X1, const float *xsc, const float *xsum,
                                                  const int *pair_tok, int bf16sim, int8_t *Hq0, int8_t *Hq1,
-                                                 float *hpart, float *hmaxp, pf_smem &sm) {
-  if (it.mcnt <= 32)
-    gate_up_tile<SHARED, 2>(L, it, nt, X0, X1, xsc, xsum, pair_tok, bf16sim, Hq0, Hq1, hpart, hmaxp, sm);
+                                                 float *hpart, float *hmaxp, pf_smem<C> &sm) {
+  if (it.mcnt <= 16)
+    gate_up_tile<C, SHARED, 1>(L, it, nt, X0, X1, xsc, xsum, pair_tok, bf16sim, Hq0, Hq1, hpart, hmaxp, sm);
+  else if (it.mcnt <= 32)
+    gate_up_tile<C, SHARED, 2>(L, it, nt, X0, X1, xsc, xsum, pair_tok, bf16sim, Hq0, Hq1, hpart, hmaxp, sm);
   else
-    gate_up_tile<SHARED, 4>(L, it, nt, X0, X1, xsc, xsum, pair_tok, bf16sim, Hq0, Hq1, hpart, hmaxp, sm);
+    gate_up_tile<C, SHARED, 4>(L, it, nt, X0, X1, xsc, xsum, pair_tok, bf16sim, Hq0, Hq1, hpart, hmaxp, sm);
 }
 
 __global__ void __launch_bounds__(256, PF_OCC) k_pf_gate_up(dsh_layer_t L, const pf_item *__restrict__ items,
@@ -954,39 +1083,41 @@ __global__ void __launch_bounds__(256, PF_OCC) k_pf_gate_up(dsh_layer_t L, const
                                                        pf_hq hq, float *__restrict__ hpr, float *__restrict__ hps,
                                                        float *__restrict__ hmr, float *__restrict__ hms,
                                                        const int *__restrict__ tiles) {
-  __shared__ __attribute__((aligned(16))) pf_smem sm;
+  typedef pf_tile_t C;
+  __shared__ __attribute__((aligned(16))) pf_smem<C> sm;
   int item, nt;
-  if (!pf_tile(counts, tiles, L.SI / PF_GU_N, L.I / PF_GU_N, item, nt)) return;
+  if (!pf_tile(counts, tiles, L.SI / C::GU, L.I / C::GU, item, nt)) return;
   const pf_item it = items[item];
   if (it.seg == L.E)
-    gate_up_dispatch<true>(L, it, nt, X0, X1, xsc, xsum, pair_tok, bf16sim, hq.s0, hq.s1, hps, hms, sm);
+    gate_up_dispatch<C, true>(L, it, nt, X0, X1, xsc, xsum, pair_tok, bf16sim, hq.s0, hq.s1, hps, hms, sm);
   else
-    gate_up_dispatch<false>(L, it, nt, X0, X1, xsc, xsum, pair_tok, bf16sim, hq.r0, hq.r1, hpr, hmr, sm);
+    gate_up_dispatch<C, false>(L, it, nt, X0, X1, xsc, xsum, pair_tok, bf16sim, hq.r0, hq.r1, hpr, hmr, sm);
 }
 
 // down: block = (work item, n-tile): the item's A rows (h of its pairs, or of tokens for the shared
-// expert, as limbs) x 256 output rows; wave w owns rows n0 + 64w .. +63 as four 16-row n-blocks. Each A
-// row's exponent is the largest of its n-tiles' (from the max |h| per (row, n-tile) the gate_up
-// epilogues wrote; read at L2); the main loop aligns every stage to it. Σh of each A row is the sum,
-// in n-tile order, of the per-n-tile row sums the gate_up epilogue wrote.
-template <bool SHARED, int MB>
+// expert, as limbs) x DN output rows; wave w owns 16·NB of them as NB 16-row n-blocks. Each A
+// row's exponent is the largest of its groups' (from the max |h| per (row, group of PF_EU units) the gate_up
+// epilogues wrote; read at L2); the main loop aligns every half stage to it. Σh of each A row is the sum,
+// in group order, of the per-group row sums the gate_up epilogue wrote.
+template <typename C, bool SHARED, int MB>
 __device__ __forceinline__ void down_tile(const dsh_layer_t &L, const pf_item &it, int nt, const int8_t *Hq0,
                                           const int8_t *Hq1, const float *hpart, const float *hmaxp, float *Y,
-                                          pf_smem &sm) {
+                                          pf_smem<C> &sm) {
+  constexpr int NB = C::NB, NE = 16 * MB * PF_NT_MAX / 256, NA = pf_arows<MB>::N;
   const int H = L.H;
-  const int Kd = SHARED ? L.SI : L.I, ntK = Kd / PF_GU_N;
+  const int Kd = SHARED ? L.SI : L.I, ntK = Kd / PF_EU;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r16 = lane & 15, kg = lane >> 4;
   const int8_t *wq = SHARED ? L.sdn_q : L.dn_q + (size_t)it.seg * H * L.I;
   const float *wso = SHARED ? L.sdn_so : L.dn_so + (size_t)it.seg * H * 2;
-  const int nw = nt * PF_DN_N + wave * 64;
+  const int nw = nt * C::DN + wave * 16 * NB;
   const size_t rbase = SHARED ? (size_t)it.m0 : (size_t)(it.pos0 + it.m0);
-  // The gate_up partials of the A rows (max |h| and Σh per row and n-tile; at most PF_MT x
-  // PF_NT_MAX = 4 per thread), read at L2 and all issued at once, then the output rows' scales
-  // and offsets; all are in flight while the main loop issues its first stage.
+  // The gate_up partials of the A rows (max |h| and Σh per row and group; at most MB·16 x
+  // PF_NT_MAX), read at L2 and all issued at once, then the output rows' scales and offsets; all are in flight
+  // while the main loop issues its first stages.
   const int ntot = it.mcnt * ntK;
-  float mxv[4], hpv[4];
+  float mxv[NE], hpv[NE];
 #pragma unroll
-  for (int c = 0; c < 4; c++) {
+  for (int c = 0; c < NE; c++) {
     const int i = threadIdx.x + 256 * c;
     mxv[c] = 0.0f;
     hpv[c] = 0.0f;
@@ -995,15 +1126,15 @@ __device__ __forceinline__ void down_tile(const dsh_layer_t &L, const pf_item &i
       hpv[c] = __hip_atomic_load(hpart + rbase * ntK + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
   }
-  float2 so[4];
+  float2 so[NB];
 #pragma unroll
-  for (int j = 0; j < 4; j++) so[j] = ((const float2 *)wso)[nw + 16 * j + r16];
-  if (threadIdx.x < PF_MT) sm.erow[threadIdx.x] = -1024;
-  // each A row's exponent (the largest of its n-tiles'), its limb scale and its Σh (n-tile order)
+  for (int j = 0; j < NB; j++) so[j] = ((const float2 *)wso)[nw + 16 * j + r16];
+  if (threadIdx.x < C::MT) sm.erow[threadIdx.x] = -1024;
+  // each A row's exponent (the largest of its groups'), its limb scale and its Σh (group order)
   auto table = [&] {
     __syncthreads();
 #pragma unroll
-    for (int c = 0; c < 4; c++) {
+    for (int c = 0; c < NE; c++) {
       const int i = threadIdx.x + 256 * c;
       if (i < ntot) {
         const int r = i / ntK, k = i - r * ntK, e = pf_limb_exp(mxv[c]);
@@ -1018,22 +1149,22 @@ __device__ __forceinline__ void down_tile(const dsh_layer_t &L, const pf_item &i
       sm.xsc[r] = __builtin_ldexpf(1.0f, sm.erow[r] - 15);
       float hs = 0.0f;
       for (int k = 0; k < ntK; k++) hs += sm.hp[r][k];
-      sm.hsum[0][r >> 5][r & 31] = hs;
+      sm.hsum[0][r] = hs;
     }
   };
-  size_t arow[2];
-  int trow[2];
+  size_t arow[NA];
+  int trow[NA];
 #pragma unroll
-  for (int c = 0; c < 2; c++) {
-    const int r = (threadIdx.x >> 3) + 32 * c;
+  for (int c = 0; c < NA; c++) {
+    const int r = pf_arows<MB>::row(c);
     trow[c] = r < it.mcnt ? r : 0;
     arow[c] = (rbase + trow[c]) * Kd;
   }
-  i32x4 acc[MB][4][2];
-  pf_mainloop_i8<MB, true>(Hq0, Hq1, arow, trow, Kd, wq + (size_t)nw * Kd, wq + (size_t)(nw + 32) * Kd, acc, sm,
-                           table);
+  i32x4 acc[MB][NB][2];
+  pf_mainloop_i8<C, MB, true>(Hq0, Hq1, arow, trow, Kd, wq + (size_t)nw * Kd, wq + (size_t)(nw + 8 * NB) * Kd, acc,
+                              sm, table);
 #pragma unroll
-  for (int j = 0; j < 4; j++) {
+  for (int j = 0; j < NB; j++) {
     const int n = nw + 16 * j + r16;
     so[j].y = __builtin_fmaf(128.0f, so[j].x, so[j].y);  // signed codes: offset + 128·scale multiplies Σh
 #pragma unroll
@@ -1042,7 +1173,7 @@ __device__ __forceinline__ void down_tile(const dsh_layer_t &L, const pf_item &i
       for (int i = 0; i < 4; i++) {
         const int m = 16 * mb + 4 * kg + i;
         if (m >= it.mcnt) continue;
-        const float hs = sm.hsum[0][m >> 5][m & 31];
+        const float hs = sm.hsum[0][m];
         // Σ q·h = 2^(erow-15)·(256·Σ q·H1 + Σ q·H0)
         const float dot = sm.xsc[m] * __builtin_fmaf(256.0f, (float)acc[mb][j][1][i], (float)acc[mb][j][0][i]);
         Y[(rbase + m) * H + n] = __builtin_fmaf(so[j].x, dot, so[j].y * hs);
@@ -1050,14 +1181,16 @@ __device__ __forceinline__ void down_tile(const dsh_layer_t &L, const pf_item &i
   }
 }
 
-template <bool SHARED>
+template <typename C, bool SHARED>
 __device__ __forceinline__ void down_dispatch(const dsh_layer_t &L, const pf_item &it, int nt, const int8_t *Hq0,
                                               const int8_t *Hq1, const float *hpart, const float *hmaxp, float *Y,
-                                              pf_smem &sm) {
-  if (it.mcnt <= 32)
-    down_tile<SHARED, 2>(L, it, nt, Hq0, Hq1, hpart, hmaxp, Y, sm);
+                                              pf_smem<C> &sm) {
+  if (it.mcnt <= 16)
+    down_tile<C, SHARED, 1>(L, it, nt, Hq0, Hq1, hpart, hmaxp, Y, sm);
+  else if (it.mcnt <= 32)
+    down_tile<C, SHARED, 2>(L, it, nt, Hq0, Hq1, hpart, hmaxp, Y, sm);
   else
-    down_tile<SHARED, 4>(L, it, nt, Hq0, Hq1, hpart, hmaxp, Y, sm);
+    down_tile<C, SHARED, 4>(L, it, nt, Hq0, Hq1, hpart, hmaxp, Y, sm);
 }
 
 __global__ void __launch_bounds__(256, PF_OCC) k_pf_down(dsh_layer_t L, const pf_item *__restrict__ items,
@@ -1066,14 +1199,15 @@ __global__ void __launch_bounds__(256, PF_OCC) k_pf_down(dsh_layer_t L, const pf
                                                     const float *__restrict__ hmr, const float *__restrict__ hms,
                                                     float *__restrict__ Y, float *__restrict__ Ysh,
                                                     const int *__restrict__ tiles) {
-  __shared__ __attribute__((aligned(16))) pf_smem sm;
+  typedef pf_tile_t C;
+  __shared__ __attribute__((aligned(16))) pf_smem<C> sm;
   int item, nt;
-  if (!pf_tile(counts, tiles, L.H / PF_DN_N, L.H / PF_DN_N, item, nt)) return;
+  if (!pf_tile(counts, tiles, L.H / C::DN, L.H / C::DN, item, nt)) return;
   const pf_item it = items[item];
   if (it.seg == L.E)
-    down_dispatch<true>(L, it, nt, hq.s0, hq.s1, hps, hms, Ysh, sm);
+    down_dispatch<C, true>(L, it, nt, hq.s0, hq.s1, hps, hms, Ysh, sm);
   else
-    down_dispatch<false>(L, it, nt, hq.r0, hq.r1, hpr, hmr, Y, sm);
+    down_dispatch<C, false>(L, it, nt, hq.r0, hq.r1, hpr, hmr, Y, sm);
 }
 
 // Fused grouped GEMM: one launch runs every gate_up and down tile, one tile per block. A block
@@ -1097,7 +1231,8 @@ __global__ void __launch_bounds__(256, PF_OCC) k_pf_moe(dsh_layer_t L, const pf_
                                                     int bf16sim, pf_hq hq, float *hpr, float *hps, float *hmr,
                                                     float *hms, float *__restrict__ Y,
                                                     float *__restrict__ Ysh) {
-  __shared__ __attribute__((aligned(16))) pf_smem sm;
+  typedef pf_tile_t C;
+  __shared__ __attribute__((aligned(16))) pf_smem<C> sm;
   __shared__ int s_tile;
   unsigned xcc;
   asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(xcc));
@@ -1111,15 +1246,15 @@ __global__ void __launch_bounds__(256, PF_OCC) k_pf_moe(dsh_layer_t L, const pf_
   const pf_item it = items[item];
   if (!(d & PF_DN_TILE)) {
     if (it.seg == L.E)
-      gate_up_dispatch<true>(L, it, nt, X0, X1, xsc, xsum, pair_tok, bf16sim, hq.s0, hq.s1, hps, hms, sm);
+      gate_up_dispatch<C, true>(L, it, nt, X0, X1, xsc, xsum, pair_tok, bf16sim, hq.s0, hq.s1, hps, hms, sm);
     else
-      gate_up_dispatch<false>(L, it, nt, X0, X1, xsc, xsum, pair_tok, bf16sim, hq.r0, hq.r1, hpr, hmr, sm);
+      gate_up_dispatch<C, false>(L, it, nt, X0, X1, xsc, xsum, pair_tok, bf16sim, hq.r0, hq.r1, hpr, hmr, sm);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this thread's limb and partial stores are in L2
     __syncthreads();
     if (threadIdx.x == 0) __hip_atomic_fetch_add(Q.gu_done + item, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   } else {
     if (threadIdx.x == 0) {
-      const int need = it.seg == L.E ? L.SI / PF_GU_N : L.I / PF_GU_N;
+      const int need = it.seg == L.E ? L.SI / C::GU : L.I / C::GU;
       int spins = 0;
       bool gave_up = Q.spin_max < 0;
       while (!gave_up && __hip_atomic_load(Q.gu_done + item, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < need) {
@@ -1133,9 +1268,9 @@ __global__ void __launch_bounds__(256, PF_OCC) k_pf_moe(dsh_layer_t L, const pf_
     }
     __syncthreads();
     if (it.seg == L.E)
-      down_dispatch<true>(L, it, nt, hq.s0, hq.s1, hps, hms, Ysh, sm);
+      down_dispatch<C, true>(L, it, nt, hq.s0, hq.s1, hps, hms, Ysh, sm);
     else
-      down_dispatch<false>(L, it, nt, hq.r0, hq.r1, hpr, hmr, Y, sm);
+      down_dispatch<C, false>(L, it, nt, hq.r0, hq.r1, hpr, hmr, Y, sm);
   }
 }
 
@@ -1253,8 +1388,8 @@ struct pf_ws {
   pf_hq hq;         // SwiGLU outputs h as int8 limbs: routed [TK][I], shared [T][SI]
   float *Y, *Ysh;
   float *ps;        // [T][4][64] router scores (DECODE: the full score in row 0, rows 1-3 zero)
-  float *hpr, *hps; // Σh partials per (row, gate_up n-tile): routed [TK][I/128], shared [T][SI/128]
-  float *hmr, *hms; // max |h| per (row, gate_up n-tile), same layout
+  float *hpr, *hps; // Σh partials per (row, group of 64 units): routed [TK][I/64], shared [T][SI/64]
+  float *hmr, *hms; // max |h| per (row, group), same layout
   int *tiles_gu, *tiles_dn;  // routed GEMM tiles (item << 8 | n-tile) in launch order
   int *qtiles, *qcount, *qnext, *gu_done, *err;  // fused kernel: work queues, counters, wait error
 };
@@ -1273,7 +1408,7 @@ int pf_grid(const dsh_layer_t *L, int T, int ntS, int ntR) {
 // Tiles one fused-kernel queue can hold: every gate_up and down tile of the largest work list.
 size_t pf_queue_cap(const dsh_layer_t *L, int T) {
   const size_t r = pf_max_routed_items(L, T), sh = pf_shared_items(T);
-  return r * (L->I / PF_GU_N) + sh * (L->SI / PF_GU_N) + (r + sh) * (L->H / PF_DN_N);
+  return r * (L->I / pf_tile_t::GU) + sh * (L->SI / pf_tile_t::GU) + (r + sh) * (L->H / pf_tile_t::DN);
 }
 
 int g_pf_xcd_min = 0;  // fewest blocks any XCD received out of a probe grid of PF_PROBE blocks
@@ -1308,12 +1443,12 @@ size_t pf_carve(const dsh_layer_t *L, int T, void *base, pf_ws *w) {
   TAKE(Y, float, TK * H);
   TAKE(Ysh, float, T * H);
   TAKE(ps, float, (size_t)T * 4 * 64);
-  TAKE(hpr, float, TK * (I / PF_GU_N));
-  TAKE(hps, float, (size_t)T * (SI / PF_GU_N));
-  TAKE(hmr, float, TK * (I / PF_GU_N));
-  TAKE(hms, float, (size_t)T * (SI / PF_GU_N));
-  TAKE(tiles_gu, int, (size_t)pf_max_routed_items(L, T) * (I / PF_GU_N));
-  TAKE(tiles_dn, int, (size_t)pf_max_routed_items(L, T) * (H / PF_DN_N));
+  TAKE(hpr, float, TK * (I / PF_EU));
+  TAKE(hps, float, (size_t)T * (SI / PF_EU));
+  TAKE(hmr, float, TK * (I / PF_EU));
+  TAKE(hms, float, (size_t)T * (SI / PF_EU));
+  TAKE(tiles_gu, int, (size_t)pf_max_routed_items(L, T) * (I / pf_tile_t::GU));
+  TAKE(tiles_dn, int, (size_t)pf_max_routed_items(L, T) * (H / pf_tile_t::DN));
   TAKE(qtiles, int, (size_t)PF_NQ * pf_queue_cap(L, T));
   TAKE(qcount, int, PF_NQ);
   TAKE(qnext, int, PF_NQ);
@@ -1327,12 +1462,11 @@ size_t pf_carve(const dsh_layer_t *L, int T, void *base, pf_ws *w) {
 extern "C" {
 
 int dsh_pf_supported(const dsh_layer_t *L) {
-  if (L->H % PF_DN_N || L->I % PF_GU_N || L->SI % PF_GU_N) return 0;
-  if (L->H % PF_KS || L->I % PF_KS || L->SI % PF_KS) return 0;
+  if (L->H % 256 || L->I % PF_KS || L->SI % PF_KS) return 0;
   if (L->E > 64 || L->K > 64 || L->K > L->E) return 0;
   if ((size_t)PF_TB * L->H * sizeof(float) > 96 * 1024) return 0;  // DECODE scores: x rows in LDS
   if (L->H > 256 * PF_SEL_U) return 0;  // a wave holds a token's x row (pf_x_limbs, k_pf_route_cfg's LDS)
-  if (L->I > PF_KS * PF_NT_MAX || L->SI > PF_KS * PF_NT_MAX) return 0;  // down: exponent table per row
+  if (L->I > PF_EU * PF_NT_MAX || L->SI > PF_EU * PF_NT_MAX) return 0;  // down: exponent table per row
   return 1;
 }
 
@@ -1450,21 +1584,28 @@ hipError_t dsh_launch_prefill(const dsh_layer_t *L, const float *X, int T, int r
   const int n_items_max = pf_max_routed_items(L, T) + pf_shared_items(T);
   const bool fused = g_pf_fused == 1 && n_items_max < (1 << 22);
   pf_queues Q{w.qtiles, w.qcount, w.qnext, w.gu_done, w.err, derr, spin_max, (int)pf_queue_cap(L, T),
-              L->I / PF_GU_N, L->SI / PF_GU_N,
-              H / PF_DN_N, H / PF_KS, L->I / PF_KS, L->SI / PF_KS, fused ? 1 : 0};
-  k_pf_plan<<<1, 1024, 0, s>>>(w.idx, T, K, E, L->I / PF_GU_N, H / PF_DN_N, w.seg_off, w.items, w.counts,
+              L->I / pf_tile_t::GU, L->SI / pf_tile_t::GU,
+              H / pf_tile_t::DN, H / PF_KS, L->I / PF_KS, L->SI / PF_KS, fused ? 1 : 0};
+  k_pf_plan<<<1, 1024, 0, s>>>(w.idx, T, K, E, L->I / pf_tile_t::GU, H / pf_tile_t::DN, w.seg_off, w.items, w.counts,
                                w.tiles_gu, w.tiles_dn, w.pair_tok, w.pos_of, Q);
   if (fused) {
-    // blocks per XCD >= tiles of the longest queue (at most ceil(items / PF_NQ) items)
-    const int per_item = max(L->I / PF_GU_N, L->SI / PF_GU_N) + H / PF_DN_N;
-    const int blocks = PF_NQ * ((n_items_max + PF_NQ - 1) / PF_NQ) * per_item;
+    // blocks per XCD >= tiles of the longest queue, whose cost is at most the mean and the costliest unit (dealt in
+    // snake order by cost); a tile costs at least the smaller of the kinds' means
+    const int nr_max = pf_max_routed_items(L, T), ns = pf_shared_items(T);
+    const int tr = Q.ngu_r + Q.ndn, ts = Q.ngu_s + Q.ndn;
+    const long cost_r = (long)Q.ngu_r * Q.nk_gu + (long)Q.ndn * Q.nk_dr;
+    const long cost_s = (long)Q.ngu_s * Q.nk_gu + (long)Q.ndn * Q.nk_ds;
+    const long unit = max(cost_s, min((long)PF_UG, (long)ns) * cost_r);
+    const long longest = (nr_max * cost_r + ns * cost_s + PF_NQ - 1) / PF_NQ + unit;
+    const long tiles = max(longest * tr / cost_r, longest * ts / cost_s) + 1;
+    const int blocks = (int)min((long)PF_NQ * tiles, (long)PF_NQ * Q.cap);
     k_pf_moe<<<blocks, 256, 0, s>>>(*L, w.items, Q, w.X0, w.X1, w.xsc, w.xsum, w.pair_tok, bf16sim, w.hq, w.hpr,
                                     w.hps, w.hmr, w.hms, w.Y, w.Ysh);
   } else {
-    k_pf_gate_up<<<pf_grid(L, T, L->SI / PF_GU_N, L->I / PF_GU_N), 256, 0, s>>>(
+    k_pf_gate_up<<<pf_grid(L, T, L->SI / pf_tile_t::GU, L->I / pf_tile_t::GU), 256, 0, s>>>(
         *L, w.items, w.counts, w.X0, w.X1, w.xsc, w.xsum, w.pair_tok, bf16sim, w.hq, w.hpr, w.hps, w.hmr, w.hms,
         w.tiles_gu);
-    k_pf_down<<<pf_grid(L, T, H / PF_DN_N, H / PF_DN_N), 256, 0, s>>>(*L, w.items, w.counts, w.hq, w.hpr, w.hps,
+    k_pf_down<<<pf_grid(L, T, H / pf_tile_t::DN, H / pf_tile_t::DN), 256, 0, s>>>(*L, w.items, w.counts, w.hq, w.hpr, w.hps,
                                                                        w.hmr, w.hms, w.Y, w.Ysh, w.tiles_dn);
   }
   k_pf_combine<<<T, 256, 0, s>>>(X, w.idx, w.w, w.pos_of, w.Y, w.Ysh, H, K, residual, bf16sim, out);

@@ -85,6 +85,29 @@ def test_prefill_small_layer(dev, B, mode, T, path):
         L.ds_hip_layer_destroy(h)
 
 
+@pytest.mark.parametrize("T", [16, 17, 32, 33, 66, 770, 1300])
+@pytest.mark.parametrize("mode", [0, 1])
+def test_prefill_uneven_experts(dev, B, mode, T):
+    """Tokens that lean the same way: a few experts get nearly all of them, the others none or a few. Item sizes around
+    the 16-, 32- and 64-row tiles, experts whose items fill several queue groups (more than eight items), experts
+    without items, and (T > 768, DECODE) the scores on the f32 MFMA. TOL covers the 16-bit activation grid, which
+    does not depend on T."""
+    L = dev.load()
+    lay = B.make_moe_layer(65, hidden=256, inter=128, n_experts=16)
+    h = upload_layer(dev, lay)
+    try:
+        X = np.stack([B.normal_f32(256, 9000 + t, std=0.3) for t in range(T)]) + 2 * B.normal_f32(256, 8999)
+        out, idx, w = gpu_prefill(dev, h, X, mode)
+        check_routing(B, lay, X, idx, w, mode)
+        n = np.bincount(idx.ravel(), minlength=16)
+        assert n.max() > T // 2 and n.min() < n.max() // 2
+        ref = np.empty((T, 256), np.float64)
+        B.oracle().or_prefill_moe_f64(ref, X, T, C.byref(lay.or_layer()), idx, w)
+        assert rel_err(out, ref) < TOL
+    finally:
+        L.ds_hip_layer_destroy(h)
+
+
 @pytest.mark.parametrize("mode", [0, 1])
 def test_prefill_one_token_equals_decode(dev, B, mode):
     """One token through the prefill block routes exactly like the decode layer and gives the same
