@@ -123,6 +123,8 @@ typedef struct {
   float *w;      /* [K] routing weights */
   float *h;      /* [K*I + SI] SwiGLU outputs (routed slots, then shared) */
   float *eo;     /* [K+1][H] expert outputs: routed slots, then shared (bf16 simulation) */
+  int *idx_out;  /* the caller's copies of idx and w [K], or NULL */
+  float *w_out;
 } dsh_layer_work_t;
 
 /* ---- prefill MoE block (k_prefill.hip) ---- */

@@ -397,6 +397,8 @@ __device__ __forceinline__ void gate_up_body(const dsh_layer_t &L, const float *
   if (blk == 0 && wave == 1 && lane < K) {  // block 0 publishes the routing (read by the down kernel)
     wk.idx[lane] = s_idx[lane];
     wk.w[lane] = s_w[lane];
+    if (wk.idx_out) wk.idx_out[lane] = s_idx[lane];  // the caller's (a copy command each costs about 2 us)
+    if (wk.w_out) wk.w_out[lane] = s_w[lane];
   }
   if (cert && blk == 0 && wave == 1 && lane == 0) cert_record(rc, s_idx, s_w, K, recomputed ? 1 : 0, x, H);
 }
@@ -628,6 +630,8 @@ __global__ void __launch_bounds__(320) k_sim_gate_up(dsh_layer_t L, const float 
   if (blockIdx.x == 0 && wave == 0 && lane < K) {
     wk.idx[lane] = s_idx[lane];
     wk.w[lane] = s_w[lane];
+    if (wk.idx_out) wk.idx_out[lane] = s_idx[lane];  // the caller's (a copy command each costs about 2 us)
+    if (wk.w_out) wk.w_out[lane] = s_w[lane];
   }
 }
 

@@ -18,8 +18,7 @@
 //                and their scale, Σx; expert selection → idx, w
 //   k_pf_scores_bf16, k_pf_select_dec  DECODE: the bf16 router's scores in the reference's AVX-512
 //                order, then the limbs and the selection
-//   k_pf_plan    expert-sorted (token, slot) pairs (stable: tokens in increasing order per expert),
-//                per-expert offsets and the GEMM work items (expert, up-to-PF_MT-row chunk)
+//   k_pf_plan    expert-sorted (token, slot) pairs, per-expert offsets and the GEMM work items (expert, up-to-PF_MT-row chunk)
 //   k_pf_gate_up grouped GEMM + SwiGLU → h as limbs, its per-(row, n-tile) sums and maxima, for
 //                routed pairs and for the shared expert
 //   k_pf_down    grouped GEMM → Y (f32) per routed pair and per token for the shared expert
@@ -33,13 +32,13 @@
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 typedef int i32x4 __attribute__((ext_vector_type(4)));
-typedef int i32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 #define PF_MT 64      // A rows per work item
 #define PF_EU 128     // intermediate units that share a limb exponent in a row of h
 #define PF_NT_MAX 16  // such groups per row of h (I, SI <= 2048)
 #define PF_TB 8     // tokens per DECODE-mode scores block
-#define PF_PLAN_LDS 8192  // (token, slot) entries the plan kernel caches in LDS
+#define PF_PLAN_LDS 65536  // (token, slot) entries the plan kernel caches in LDS (a byte each)
 #define PF_NQ 8           // work queues of the fused GEMM kernel: one per XCD
 #define PF_UG 8           // items of one expert that share a queue, at most
 #define PF_DN_TILE 0x80000000u  // tile word: down tile flag | item << 8 | n-tile
@@ -139,7 +138,7 @@ __global__ void __launch_bounds__(256) k_pf_route_cfg(const float *__restrict__ 
                                                       int T, int H, int E, int K, int8_t *__restrict__ X0,
                                                       int8_t *__restrict__ X1, float *__restrict__ xsc,
                                                       float *__restrict__ xsum, int *__restrict__ idx,
-                                                      float *__restrict__ w) {
+                                                      float *__restrict__ w, int *idx_out, float *w_out) {
   __shared__ __attribute__((aligned(16))) float s_wr[2][PF_RC_KC * 64];
   __shared__ __attribute__((aligned(16))) float s_x[4][256 * PF_SEL_U];
   __shared__ float s_red[4][4][64];
@@ -277,6 +276,8 @@ __global__ void __launch_bounds__(256) k_pf_route_cfg(const float *__restrict__ 
   if (own && lane < K) {
     idx[(size_t)t * K + lane] = s_idx[wave][lane];
     w[(size_t)t * K + lane] = s_w[wave][lane];
+    if (idx_out) idx_out[(size_t)t * K + lane] = s_idx[wave][lane];  // the caller's (a copy command each costs 3-5 us)
+    if (w_out) w_out[(size_t)t * K + lane] = s_w[wave][lane];
   }
 }
 // DECODE (bf16 router in the reference's AVX-512 order, as k_dec_scores_bf16): one block per PF_TB
@@ -358,13 +359,134 @@ __global__ void __launch_bounds__(256) k_pf_scores_bf16r(const uint16_t *__restr
   }
 }
 
+// The same scores on the f32 MFMA, for many tokens: v_mfma_f32_16x16x1 adds one rounded-once product to each of its
+// accumulators (the bits of fmaf, subnormals included), so a chain of the reference's order is a chain of
+// MFMAs over its columns. A block takes 16 tokens x 64 experts; wave v runs chains 8v .. 8v+7 (columns
+// 32i + 8v + c), four 16-expert blocks per instruction, 16 accumulators per chain and lane. Router rows and
+// tokens pass through LDS 128 columns at a time (swizzled 16-byte pieces), the next ones on their way in registers.
+// Then the order's own sums: a0 + a1 (waves 0 + 2, 1 + 3), T3 (waves 0 + 1), T6 and the last pair.
+// 18.5 us at 3001 tokens; k_pf_scores_bf16r, which unpacks a row and reads x from LDS for every token, takes 46.5.
+#define PF_SM_T 16
+struct pf_scores_smem {
+  union {
+    struct {
+      u32x4 w[64][16];           // 64 router rows x 128 bf16 columns
+      f32x4 x[PF_SM_T][32];      // 16 tokens x 128 columns
+    } s[2];
+    f32x4 a[2][8][4][64];        // chain sums of two waves: [wave][chain][register / 4][lane]
+  };
+};
+__global__ void __launch_bounds__(256, 2) k_pf_scores_mfma(const uint16_t *__restrict__ Wr, const float *__restrict__ X,
+                                                        int T, int H, int E, float *__restrict__ ps) {
+  __shared__ __attribute__((aligned(16))) pf_scores_smem S;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r16 = lane & 15;
+  const int t0 = blockIdx.x * PF_SM_T, nst = H / 128;
+  u32x4 wr[4];
+  f32x4 xr[2];
+  auto load = [&](int st) {  // 16 lanes per router row's 256 bytes, 32 per token row's 512
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+      wr[i] = ((const u32x4 *)(Wr + (size_t)min((tid >> 4) + 16 * i, E - 1) * H + 128 * st))[tid & 15];
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+      xr[i] = ((const f32x4 *)(X + (size_t)min(t0 + (tid >> 5) + 8 * i, T - 1) * H + 128 * st))[tid & 31];
+  };
+  auto store = [&](int b) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const int r = (tid >> 4) + 16 * i;
+      S.s[b].w[r][(tid & 15) ^ (r & 15)] = wr[i];
+    }
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      const int r = (tid >> 5) + 8 * i;
+      S.s[b].x[r][(tid & 31) ^ r] = xr[i];
+    }
+  };
+  f32x16 acc[8];
+#pragma unroll
+  for (int c = 0; c < 8; c++)
+#pragma unroll
+    for (int i = 0; i < 16; i++) acc[c][i] = 0.0f;
+  load(0);
+  store(0);
+#pragma unroll 1
+  for (int st = 0; st < nst; st++) {
+    const int b = st & 1;
+    load(min(st + 1, nst - 1));
+    __syncthreads();
+    u32x4 w[2];
+    f32x4 x[2][2];
+    auto rd = [&](int i) {  // columns 128 st + 32 i + 8 wave .. + 7
+      w[i & 1] = S.s[b].w[lane][(4 * i + wave) ^ r16];
+      x[i & 1][0] = S.s[b].x[r16][(8 * i + 2 * wave) ^ r16];
+      x[i & 1][1] = S.s[b].x[r16][(8 * i + 2 * wave + 1) ^ r16];
+    };
+    rd(0);
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      if (i < 3) rd(i + 1);  // read while the MFMAs of i run
+      __builtin_amdgcn_sched_barrier(0);
+      float wf[8];
+#pragma unroll
+      for (int c = 0; c < 8; c++) wf[c] = c & 1 ? dsh_bf16hi(w[i & 1][c >> 1]) : dsh_bf16lo(w[i & 1][c >> 1]);
+#pragma unroll
+      for (int c = 0; c < 8; c++)
+        acc[c] = __builtin_amdgcn_mfma_f32_16x16x1f32(x[i & 1][c >> 2][c & 3], wf[c], acc[c], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    store(b ^ 1);  // the other buffer: every wave was done with it before the last barrier
+  }
+  __syncthreads();
+  auto put = [&](f32x4 (*a)[4][64]) {
+#pragma unroll
+    for (int c = 0; c < 8; c++)
+#pragma unroll
+      for (int q = 0; q < 4; q++)
+        a[c][q][lane] = f32x4{acc[c][4 * q], acc[c][4 * q + 1], acc[c][4 * q + 2], acc[c][4 * q + 3]};
+  };
+  auto add = [&](const f32x4 (*a)[4][64]) {
+#pragma unroll
+    for (int c = 0; c < 8; c++)
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const f32x4 v = a[c][q][lane];
+#pragma unroll
+        for (int i = 0; i < 4; i++) acc[c][4 * q + i] += v[i];
+      }
+  };
+  if (wave >= 2) put(S.a[wave - 2]);
+  __syncthreads();
+  if (wave < 2) add(S.a[wave]);  // a0 + a1: chains 8 wave .. 8 wave + 7 of 16
+  __syncthreads();
+  if (wave == 1) put(S.a[0]);
+  __syncthreads();
+  if (wave != 0) return;
+  add(S.a[0]);  // T3
+#pragma unroll
+  for (int i = 0; i < 16; i++) {  // token 4 (lane / 16) + i % 4, expert 16 (i / 4) + lane % 16
+    float t6[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) t6[j] = acc[4 + j][i] + acc[j][i];
+    const float v = ((t6[0] + t6[2]) + (t6[1] + t6[3])) + 0.0f;
+    const int t = t0 + 4 * (lane >> 4) + (i & 3), e = 16 * (i >> 2) + r16;
+    if (t < T) {
+      float *o = ps + (size_t)t * 4 * 64 + e;
+      o[0] = e < E ? v : 0.0f;
+      o[64] = 0.0f;
+      o[128] = 0.0f;
+      o[192] = 0.0f;
+    }
+  }
+}
+
 // DECODE: one wave per token, x's limbs (pf_x_limbs), then the fast-exp softmax over all experts
 // and top-k (route_select) on the scores of k_pf_scores_bf16.
 __global__ void __launch_bounds__(256) k_pf_select_dec(const float *__restrict__ X, int T, int H, int E, int K,
                                                        const float *__restrict__ ps, int8_t *__restrict__ X0,
                                                        int8_t *__restrict__ X1, float *__restrict__ xsc,
                                                        float *__restrict__ xsum, int *__restrict__ idx,
-                                                       float *__restrict__ w) {
+                                                       float *__restrict__ w, int *idx_out, float *w_out) {
   __shared__ float s_red[4][4][64];
   __shared__ int s_idx[4][64];
   __shared__ float s_w[4][64];
@@ -381,16 +503,17 @@ __global__ void __launch_bounds__(256) k_pf_select_dec(const float *__restrict__
   if (lane < K) {
     idx[(size_t)t * K + lane] = s_idx[wave][lane];
     w[(size_t)t * K + lane] = s_w[wave][lane];
+    if (idx_out) idx_out[(size_t)t * K + lane] = s_idx[wave][lane];  // the caller's (a copy command each costs 3-5 us)
+    if (w_out) w_out[(size_t)t * K + lane] = s_w[wave][lane];
   }
 }
 
 // ---------------------------------------------------------------------------------- plan
-// One 1024-thread block. Wave v owns a contiguous range of the T·K (token, slot) entries. Per-wave
+// One 1024-thread block. Its time is a chain of round trips (5-8 us up to 662 tokens): the entries come from memory once
+// (a byte each in LDS: read again from memory for each 64 they took 16 of 24 us at 3001 tokens). Wave v owns a contiguous range of the T·K (token, slot) entries. Per-wave
 // expert counts give each expert's segment offset and each wave's start inside it, so a pair's
 // position is (segment offset) + (pairs of the expert in earlier waves) + (earlier pairs of the
-// expert in this wave): expert segments hold their tokens in increasing order. Within a wave, 64
-// entries at a time, the entries routed to the same expert are found with 7 ballots over the
-// expert's bits. Entries with no expert (idx < 0 or >= E) get pos_of = -1.
+// expert in this wave). Entries with no expert (idx < 0 or >= E) get pos_of = -1.
 // Work items: each expert's pairs in chunks of PF_MT (items 0 .. n_routed-1), then the shared
 // expert's T tokens in chunks of PF_MT; counts = {n_routed, n_shared}; and the routed GEMM tile
 // lists of both projections.
@@ -405,7 +528,7 @@ __global__ void __launch_bounds__(1024) k_pf_plan(const int *__restrict__ idx, i
   __shared__ int s_ucls[PF_UG + 1][64], s_utot[PF_UG + 1];  // queue units by size: before expert e, in all
   __shared__ int s_qgu[PF_NQ][PF_UG + 1], s_qdn[PF_NQ][PF_UG + 1];
   __shared__ int run[16][64];
-  __shared__ int cache[PF_PLAN_LDS];
+  __shared__ unsigned char cache[PF_PLAN_LDS];  // the entries' experts, 255: none
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int TK = T * K;
   const bool cached = TK <= PF_PLAN_LDS;
@@ -421,17 +544,30 @@ __global__ void __launch_bounds__(1024) k_pf_plan(const int *__restrict__ idx, i
     for (int u = 0; u < 8; u++) {
       const int i = base + 64 * u + lane;
       if (i >= hi) continue;
-      if (cached) cache[i] = ev[u];
-      if (ev[u] >= 0 && ev[u] < E) atomicAdd(&cnt[wave][ev[u]], 1);
+      const bool valid = ev[u] >= 0 && ev[u] < E;
+      if (cached) cache[i] = (unsigned char)(valid ? ev[u] : 255);
+      if (valid) atomicAdd(&cnt[wave][ev[u]], 1);
     }
   }
   __syncthreads();
-  if (wave == 0) {  // lane = expert
-    int cv[16], c = 0;  // the waves' counts, all read before the prefix
+  int cv[16], c = 0;  // lane = expert: the waves' counts, all read before the prefix
 #pragma unroll
-    for (int v = 0; v < 16; v++) cv[v] = lane < E ? cnt[v][lane] : 0;
+  for (int v = 0; v < 16; v++) cv[v] = lane < E ? cnt[v][lane] : 0;
 #pragma unroll
-    for (int v = 0; v < 16; v++) c += cv[v];
+  for (int v = 0; v < 16; v++) c += cv[v];
+  if (Q.enable && wave >= 1 && wave <= PF_UG) {  // wave v counts the queue units (below) of v items
+    const int nch = (c + PF_MT - 1) / PF_MT, ug = (nch + PF_UG - 1) / PF_UG, sz = ug ? nch / ug : 0, big = nch - sz * ug;
+    const int n = wave == sz ? ug - big : (wave == sz + 1 ? big : 0);
+    int incl = n;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int o = __shfl_up(incl, d);
+      if (lane >= d) incl += o;
+    }
+    s_ucls[wave][lane] = incl - n;
+    if (lane == 63) s_utot[wave] = incl;
+  }
+  if (wave == 0) {
     int incl = c;
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
@@ -489,19 +625,6 @@ __global__ void __launch_bounds__(1024) k_pf_plan(const int *__restrict__ idx, i
     // tiles, then its down tiles, in rank order. Ranks and offsets have closed forms.
     const int ns = (T + PF_MT - 1) / PF_MT, nr = s_nr, nu = nr + ns;
     const int cost_s = Q.ngu_s * Q.nk_gu + Q.ndn * Q.nk_ds, cost_r = Q.ngu_r * Q.nk_gu + Q.ndn * Q.nk_dr;
-    if (wave < PF_UG) {  // wave v counts the groups of v + 1 items, lane = expert
-      const int nch = s_nch[lane], ug = (nch + PF_UG - 1) / PF_UG, sz = ug ? nch / ug : 0, big = nch - sz * ug;
-      const int c = wave + 1 == sz ? ug - big : (wave + 1 == sz + 1 ? big : 0);
-      int incl = c;
-#pragma unroll
-      for (int d = 1; d < 64; d <<= 1) {
-        const int o = __shfl_up(incl, d);
-        if (lane >= d) incl += o;
-      }
-      s_ucls[wave + 1][lane] = incl - c;
-      if (lane == 63) s_utot[wave + 1] = incl;
-    }
-    __syncthreads();
     // rank ranges: classes of routed groups by size, large first, the shared items (class 0) where their cost puts them
     int st[PF_UG + 1], tot[PF_UG + 1];
     {
@@ -594,24 +717,15 @@ __global__ void __launch_bounds__(1024) k_pf_plan(const int *__restrict__ idx, i
       for (int nt = 0; nt < Q.ndn; nt++) qt[dn0 + nt * m + j] = (int)(PF_DN_TILE | (u << 8) | nt);
     }
   }
-  // the pair positions (no barrier: they read only run and the cached entries, both complete)
+  // The pair positions (no barrier: they read only run and the cached entries, both complete). Within 64 entries an
+  // expert's pairs take the order of the LDS atomics; no output depends on it (a pair's row is computed by itself and
+  // found again through pos_of). Ranked by ballots over the expert's bits instead, 64 entries take some 100
+  // instructions of a wave, 12 us at 3001 tokens.
   for (int base = lo; base < hi; base += 64) {
     const int i = base + lane;
-    const int e = i < hi ? (cached ? cache[i] : idx[i]) : -1;
+    const int e = i < hi ? (cached ? (int)cache[i] : idx[i]) : -1;
     const bool valid = e >= 0 && e < E;
-    const int key = valid ? e : 127;
-    unsigned long long same = ~0ull;
-#pragma unroll
-    for (int b = 0; b < 7; b++) {
-      const bool bit = (key >> b) & 1;
-      const unsigned long long m = __ballot(bit);
-      same &= bit ? m : ~m;
-    }
-    const int rank = __popcll(same & ((1ull << lane) - 1ull));
-    const int p = valid ? run[wave][e] + rank : -1;
-    __builtin_amdgcn_wave_barrier();
-    if (valid && rank == 0) run[wave][e] = p + __popcll(same);
-    __builtin_amdgcn_wave_barrier();
+    const int p = valid ? atomicAdd(&run[wave][e], 1) : -1;
     if (i < hi) {
       if (valid) pair_tok[p] = i / K;
       pos_of[i] = p;
@@ -785,7 +899,7 @@ hipError_t dsh_launch_pf_swiglu_check(unsigned long long *counts, hipStream_t s)
 // distinct bank groups, and two consecutive rows fill 256 contiguous bytes
 __device__ __forceinline__ int pf_swz(int r) { return (r ^ (r >> 3)) & 7; }
 
-// Stages of loads in flight per wave: A and B registers of a stage are reloaded with the stage D later once they
+// Stages of loads in flight per wave (what the registers allow beside 32 MB accumulators): A and B registers of a stage are reloaded with the stage D later once they
 // are used. A wave's loads return in issue order, so A runs as far ahead as B: an A stage loaded one
 // stage ahead would wait for every weight load issued before it.
 constexpr int pf_depth(int MB) { return MB == 1 ? 3 : (MB == 2 ? 2 : 1); }
@@ -794,7 +908,7 @@ constexpr int pf_depth(int MB) { return MB == 1 ? 3 : (MB == 2 ? 2 : 1); }
 // - weights go from HBM straight into the MFMA's B operand registers: for n-block j (16 weight
 //   rows: the first NB/2 from brow0, the others from brow1) and slice s, lane l loads bytes 64s + 16(l/16) .. +15
 //   of the stage in row 16j + l%16 (each load instruction reads 16 rows x 64 contiguous bytes; the two slices' loads
-//   are issued together, so the second finds its lines on their way);
+//   are issued together: half a stage apart the L1 had lost the line, and 1.5 times the lines came from L2);
 // - A: the block's rows are copied (8 adjacent lanes per row's 128 bytes) into a double-buffered LDS tile with
 //   128-byte rows whose 16-byte chunks are XOR-swizzled by pf_swz(row); lane l reads chunk 4s + l/16 of
 //   row 16mb + l%16, the same columns as its weight bytes, so each MFMA adds the exact products over the
@@ -1558,10 +1672,10 @@ hipError_t dsh_launch_prefill(const dsh_layer_t *L, const float *X, int T, int r
   if (route_mode == DSH_ROUTE_CFG) {
     if (E == 64)
       k_pf_route_cfg<true><<<(T + 3) / 4, 256, 0, s>>>(L->router_f32_t, X, T, H, E, K, w.X0, w.X1, w.xsc, w.xsum,
-                                                        w.idx, w.w);
+                                                        w.idx, w.w, idx_out, w_out);
     else
       k_pf_route_cfg<false><<<(T + 3) / 4, 256, 0, s>>>(L->router_f32_t, X, T, H, E, K, w.X0, w.X1, w.xsc, w.xsum,
-                                                         w.idx, w.w);
+                                                         w.idx, w.w, idx_out, w_out);
   } else {
     // every row on a group path: the chunks of the reference's threads all have an even length
     const int chunk = dsh_chunk_len(E, nthreads);
@@ -1572,14 +1686,19 @@ hipError_t dsh_launch_prefill(const dsh_layer_t *L, const float *X, int T, int r
   case N:                                                                                                           \
     k_pf_scores_bf16r<N><<<nbr, 256, 0, s>>>(L->router_bf16, X, T, E, tpb, w.ps);                                 \
     break;
-    if (grouped && H % 256 == 0 && H <= 1280) {
+    // the MFMA kernel takes one pass whatever the tokens (up to 8192: two blocks per CU; 18.5 us at 3001), the one with
+    // the rows in registers a pass per token of a block (7 us with one, 14.5 with three, 46.5 with twelve)
+    if (grouped && H % 256 == 0 && (tpb > 3 || H > 1280)) {
+      k_pf_scores_mfma<<<(T + PF_SM_T - 1) / PF_SM_T, 256, 0, s>>>(L->router_bf16, X, T, H, E, w.ps);
+    } else if (grouped && H % 256 == 0) {
       switch (H / 32) { PFR(8) PFR(16) PFR(24) PFR(32) PFR(40) }
     } else {
       k_pf_scores_bf16<<<(T + PF_TB - 1) / PF_TB, 256, (size_t)PF_TB * H * sizeof(float), s>>>(
           L->router_bf16, X, T, H, E, nthreads, w.ps);
     }
 #undef PFR
-    k_pf_select_dec<<<(T + 3) / 4, 256, 0, s>>>(X, T, H, E, K, w.ps, w.X0, w.X1, w.xsc, w.xsum, w.idx, w.w);
+    k_pf_select_dec<<<(T + 3) / 4, 256, 0, s>>>(X, T, H, E, K, w.ps, w.X0, w.X1, w.xsc, w.xsum, w.idx, w.w, idx_out,
+                                                     w_out);
   }
   const int n_items_max = pf_max_routed_items(L, T) + pf_shared_items(T);
   const bool fused = g_pf_fused == 1 && n_items_max < (1 << 22);
@@ -1609,12 +1728,7 @@ hipError_t dsh_launch_prefill(const dsh_layer_t *L, const float *X, int T, int r
                                                                        w.hmr, w.hms, w.Y, w.Ysh, w.tiles_dn);
   }
   k_pf_combine<<<T, 256, 0, s>>>(X, w.idx, w.w, w.pos_of, w.Y, w.Ysh, H, K, residual, bf16sim, out);
-  hipError_t e = hipGetLastError();
-  if (e == hipSuccess && idx_out)
-    e = hipMemcpyAsync(idx_out, w.idx, sizeof(int) * (size_t)T * K, hipMemcpyDeviceToDevice, s);
-  if (e == hipSuccess && w_out)
-    e = hipMemcpyAsync(w_out, w.w, sizeof(float) * (size_t)T * K, hipMemcpyDeviceToDevice, s);
-  return e;
+  return hipGetLastError();
 }
 
 }  // extern "C"

@@ -326,13 +326,12 @@ int ds_hip_layer_forward(ds_hip_layer_t *L, float *out_dev, const float *x_dev, 
   if (!L || !out_dev || !x_dev) return dsr_failf("ds_hip_layer_forward: NULL argument");
   if (check_router(L, route_mode)) return -1;
   int bf16sim = ds_bf16_simulate_python;
-  hipError_t e = layer_enqueue(L, &L->wk, L->partials, 0, 0, x_dev, NULL, 0, out_dev, route_mode, residual, bf16sim,
+  dsh_layer_work_t wk = L->wk;
+  wk.idx_out = idx_dev; /* written by the kernel that selects, which keeps its own for the next one */
+  wk.w_out = w_dev;
+  hipError_t e = layer_enqueue(L, &wk, L->partials, 0, 0, x_dev, NULL, 0, out_dev, route_mode, residual, bf16sim,
                                NULL, NULL, NULL);
   if (e != hipSuccess) return dsr_fail("layer kernels", e);
-  if (idx_dev)
-    DSR_TRY(hipMemcpyAsync(idx_dev, L->wk.idx, (size_t)L->K * 4, hipMemcpyDeviceToDevice, dsr_stream), "idx copy");
-  if (w_dev)
-    DSR_TRY(hipMemcpyAsync(w_dev, L->wk.w, (size_t)L->K * 4, hipMemcpyDeviceToDevice, dsr_stream), "w copy");
   return 0;
 }
 
@@ -374,7 +373,7 @@ int ds_hip_layer_prefill(ds_hip_layer_t *L, float *out_dev, const float *x_dev, 
   key.fused = dsh_pf_fused();
   key.spin_max = g_pf_spin_max;
   if (!L->pf_exec || memcmp(&key, &L->pf_key, sizeof key) != 0) {
-    /* the seven kernels (and the idx/w copies) captured once, then one graph launch per call */
+    /* the kernels captured once, then one graph launch per call */
     if (L->pf_exec) { /* an earlier call's launch of it may still run on the stream */
       DSR_TRY(hipStreamSynchronize(dsr_stream), "prefill graph");
       hipGraphExecDestroy(L->pf_exec);
