@@ -332,3 +332,31 @@ def test_linear_bf16_batched(dev, B):
     L.ds_linear_nobias_bf16(Y, X, W, M, K, N)
     ref = X.reshape(M, K).astype(np.float64) @ B.bf16_to_f32(W).reshape(N, K).astype(np.float64).T
     assert rel_err(Y.reshape(M, N), ref) < 1e-5
+
+
+@pytest.mark.parametrize("M,K,N", [(2, 1, 1), (3, 7, 5), (64, 64, 64), (65, 72, 130), (63, 63, 65), (130, 1985, 70),
+                                   (662, 1280, 96)])
+@pytest.mark.parametrize("scale", [1.0, 1e-30, 1e30])
+def test_linear_bf16_batched_shapes(dev, B, M, K, N, scale):
+    """Tile edges, odd K (rows that are not aligned) and magnitudes near both ends of f32. Every product is exact, so an
+    element differs from f64 by the roundings of its sum: at most K + 3 of them (2^-24 each) on any partial sum,
+    which is at most the sum of |x w|. Infinities and NaN: the same classes as f64 gives."""
+    L = dev.load()
+    X = (B.normal_f32(M * K, 410 + K) * np.float32(scale)).reshape(M, K)
+    W = B.normal_bf16(N * K, 411 + K, 0.05)
+    Y = np.empty(M * N, np.float32)
+    L.ds_linear_nobias_bf16(Y, X.reshape(-1), W, M, K, N)
+    W64 = B.bf16_to_f32(W).reshape(N, K).astype(np.float64)
+    ref, size = X.astype(np.float64) @ W64.T, np.abs(X).astype(np.float64) @ np.abs(W64.T)
+    assert np.all(np.abs(Y.reshape(M, N) - ref) <= (K + 3) * 2.0 ** -24 * size)
+    X[0, 0], X[M - 1, K - 1] = np.inf, np.nan
+    W2 = W.copy()  # a new array: registered weights are not edited
+    W2[(N - 1) * K] = 0x7F80
+    L.ds_linear_nobias_bf16(Y, X.reshape(-1), W2, M, K, N)
+    L.ds_hip_weights_changed(W2.ctypes.data)  # both arrays go now; another may come to lie at their addresses
+    L.ds_hip_weights_changed(W.ctypes.data)
+    with np.errstate(invalid="ignore", over="ignore"):
+        ref = X.astype(np.float64) @ B.bf16_to_f32(W2).reshape(N, K).astype(np.float64).T
+    got = Y.reshape(M, N)
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    assert np.array_equal(np.isinf(got), np.isinf(ref)) and np.array_equal(got[np.isinf(got)], ref[np.isinf(got)])
