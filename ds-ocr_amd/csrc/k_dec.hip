@@ -552,80 +552,198 @@ __global__ void __launch_bounds__(512) k_dec_down(dsh_layer_t L, const float *__
 // With ds_bf16_simulate_python the reference rounds gate, up, the SwiGLU output and every expert's
 // output to bf16 (ds_quantize.c:311-320). A value summed in any order other than the reference's
 // lands on the other side of a rounding boundary now and then, so these kernels compute every
-// rounded value in the reference's own order (dsh_row_chain: one lane per row, the row's
-// sequential fused chain, ds_quantize.c:163-166; Σx and Σh as sequential sums): for the same routing
-// the layer output is bit-identical to the reference's. One lane per row makes them latency-bound
-// (one 1280-long chain per projection); the unrounded mode keeps the fast kernels above.
+// rounded value in the reference's own order (one lane per row, the row's sequential fused chain,
+// ds_quantize.c:163-166: dot = fma(u_j, x_j, dot), j ascending; Σx and Σh as sequential sums): for the same
+// routing the layer output is bit-identical to the reference's. The chains bound them (one of 1280 steps, then one of
+// 896 or 1792 dependent fused multiply-adds); the unrounded mode keeps the fast kernels above.
 //
-// k_sim_gate_up: block b owns units 128b .. 128b+127 (the routed units k*I + i, then the shared
-// expert's); threads 0-127 run the units' gate rows, 128-255 their up rows, and lane 0 of a fifth
-// wave sums x. Waves 0-3 route as k_dec_gate_up does (each for itself). h = bf16(SwiGLU(bf16(g),
-// bf16(u))); block 0 publishes the routing.
-__global__ void __launch_bounds__(320) k_sim_gate_up(dsh_layer_t L, const float *x_in, const int *__restrict__ step,
-                                                     int stride, const float *partials, int np, int mode,
-                                                     dsh_layer_work_t wk) {
+// sim_rows: 64 rows per block of SIM_THREADS threads, n columns (a multiple of 16) in chunks of 128. Waves 0-3 copy the
+// rows' codes to LDS as f32 (exact), 8 adjacent lanes per row, SIM_D chunks of loads in flight; wave 4 runs the
+// chains (lane = row) a chunk behind them; wave 5 adds up x. A step of a chain is one instruction, its x taken from
+// 16 lanes that hold 16 columns (row_newbcast), and costs the 8.7 clocks that the next one waits for it; a code widened
+// in the step takes 13.5 (from a byte) or 15.4 (v_fma_mix_f32). One lane per row reading its row itself, 16 bytes of 64
+// lines per load, took 46.7 and 21.9 us for the two kernels below at DeepSeek-OCR's shape (1280, 896, shared 1792),
+// v_fma_mix_f32 with x read by every lane 17.2 and 18.0, two chunks in LDS instead of three (no operands read ahead
+// across a chunk's end) 15.1 and 14.5; now 14.3 and 12.3.
+// x: n floats in LDS, written by waves 4 and 5 or before the caller's last barrier; row(r): the first code of row r
+// (0..63). Returns the lane's dot in wave 4, Σx in wave 5.
+#define SIM_THREADS 384
+#define SIM_D 6  // a multiple of 3
+#define SIM_KC 128
+struct sim_smem {
+  __attribute__((aligned(16))) float q[3][64][SIM_KC + 4];
+};
+// Four stored codes (u - 128 as bytes) to u.
+__device__ __forceinline__ f32x4 sim_codes(unsigned w) {
+  w ^= 0x80808080u;
+  return f32x4{(float)(w & 255), (float)(w >> 8 & 255), (float)(w >> 16 & 255), (float)(w >> 24)};
+}
+// 16 steps: acc = fma(q_e, x_e, acc), or acc + x_e with SUM; lane e of every 16 holds x_e in v. In assembly, as the
+// compiler puts s_nop 1 between the steps: only a DPP operand (v, from LDS) must not come from the two instructions
+// before, which the one s_nop here covers.
+#define SIM_BC(e) " row_newbcast:" #e " row_mask:0xf bank_mask:0xf\n"
+#define SIM_FMA(e, q) "v_fmac_f32_dpp %0, %1, %" #q SIM_BC(e)
+#define SIM_ADD(e) "v_add_f32_dpp %0, %1, %0" SIM_BC(e)
+template <bool SUM>
+__device__ __forceinline__ float sim_steps(float acc, const f32x4 *q, float v) {
+  if (SUM)
+    asm volatile("s_nop 1\n" SIM_ADD(0) SIM_ADD(1) SIM_ADD(2) SIM_ADD(3) SIM_ADD(4) SIM_ADD(5) SIM_ADD(6) SIM_ADD(7)
+                     SIM_ADD(8) SIM_ADD(9) SIM_ADD(10) SIM_ADD(11) SIM_ADD(12) SIM_ADD(13) SIM_ADD(14) SIM_ADD(15)
+                 : "+v"(acc)
+                 : "v"(v));
+  else
+    asm volatile("s_nop 1\n" SIM_FMA(0, 2) SIM_FMA(1, 3) SIM_FMA(2, 4) SIM_FMA(3, 5) SIM_FMA(4, 6) SIM_FMA(5, 7)
+                     SIM_FMA(6, 8) SIM_FMA(7, 9) SIM_FMA(8, 10) SIM_FMA(9, 11) SIM_FMA(10, 12) SIM_FMA(11, 13)
+                         SIM_FMA(12, 14) SIM_FMA(13, 15) SIM_FMA(14, 16) SIM_FMA(15, 17)
+                 : "+v"(acc)
+                 : "v"(v), "v"(q[0][0]), "v"(q[0][1]), "v"(q[0][2]), "v"(q[0][3]), "v"(q[1][0]), "v"(q[1][1]),
+                   "v"(q[1][2]), "v"(q[1][3]), "v"(q[2][0]), "v"(q[2][1]), "v"(q[2][2]), "v"(q[2][3]), "v"(q[3][0]),
+                   "v"(q[3][1]), "v"(q[3][2]), "v"(q[3][3]));
+  return acc;
+}
+// The dots or, with SUM, the sum of x in element order (every lane the same). Operands are read two pieces of 16
+// columns ahead, across the chunks: a chunk starts when the next one is in LDS too.
+template <bool SUM>
+__device__ __forceinline__ float sim_chain(const sim_smem &S, const float *x, int n) {
+  const int lane = threadIdx.x & 63, nch = (n + SIM_KC - 1) / SIM_KC;
+  constexpr int P = SIM_KC / 16;
+  float acc = 0.0f;
+  f32x4 q[4][4];
+  float v[4];
+  const float *q0 = &S.q[0][lane][0], *q1 = &S.q[1][lane][0];  // a chunk's codes and the next one's
+  auto ld = [&](int k, int c, const float *qc, int i) {  // piece i of chunk c; past the end: the last x again, not used
+    v[k] = x[min(SIM_KC * c + 16 * i, n - 16) + (lane & 15)];
+    if (!SUM) {
+      qc += 16 * i;
+#pragma unroll
+      for (int d = 0; d < 4; d++) q[k][d] = *(const f32x4 *)(qc + 4 * d);
+    }
+  };
+  auto step = [&](int k) {
+    __builtin_amdgcn_sched_barrier(0);
+    acc = sim_steps<SUM>(acc, q[k], v[k]);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  __builtin_amdgcn_s_setprio(3);  // the chains go first on their SIMDs
+  __syncthreads();
+  ld(0, 0, q0, 0);
+  ld(1, 0, q0, 1);
+  for (int c = 0; c < nch - 1; c++) {
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < P; i++) {
+      ld((i + 2) % 4, c + (i + 2) / P, i + 2 < P ? q0 : q1, (i + 2) % P);
+      step(i % 4);
+    }
+    q0 = q1;
+    q1 = q1 == &S.q[2][lane][0] ? &S.q[0][lane][0] : q1 + 64 * (SIM_KC + 4);
+  }
+  const int m = (n - SIM_KC * (nch - 1)) / 16;  // pieces of the last chunk
+#pragma unroll
+  for (int i = 0; i < P; i++) {
+    if (i >= m) break;
+    if (i + 2 < P) ld((i + 2) % 4, nch - 1, q0, i + 2);
+    step(i % 4);
+  }
+  __builtin_amdgcn_s_setprio(0);
+  return acc;
+}
+template <typename Row>
+__device__ __forceinline__ float sim_rows(sim_smem &S, const float *x, int n, Row &&row) {
+  const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  if (wave == 4) return sim_chain<false>(S, x, n);
+  if (wave == 5) return sim_chain<true>(S, x, n);
+  const int nch = (n + SIM_KC - 1) / SIM_KC;
+  const int8_t *p[2];
+  u32x4 v[SIM_D][2];
+#pragma unroll
+  for (int j = 0; j < 2; j++) p[j] = row((t >> 3) + 32 * j);
+  auto load = [&](int d, int c) {
+    const int o = min(SIM_KC * c + 16 * (t & 7), n - 16);  // past the end: the last codes again, not used
+#pragma unroll
+    for (int j = 0; j < 2; j++) v[d][j] = dsh_load_nt(p[j] + o);
+    asm volatile("" ::: "memory");
+  };
+#pragma unroll
+  for (int d = 0; d < SIM_D; d++) load(d, d);
+  auto stage = [&](int d, int c) {
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+      f32x4 *at = (f32x4 *)&S.q[d % 3][(t >> 3) + 32 * j][16 * (t & 7)];
+      const int b = t >> 2 & 1;  // 8 lanes' 16 bytes on different banks
+#pragma unroll
+      for (int i = 0; i < 4; i++) at[i ^ b] = sim_codes(b ? v[d][j][i ^ 1] : v[d][j][i]);
+    }
+    __builtin_amdgcn_sched_barrier(0);  // the next load takes this one's registers
+    load(d, c + SIM_D);
+    __builtin_amdgcn_sched_barrier(0);  // no later chunk's codes are waited for here
+    __syncthreads();  // chunk c is in LDS; wave 4 is done with chunk c - 2, whose buffer the next one takes
+  };
+  int c = 0;
+  for (; c + SIM_D <= nch; c += SIM_D) {
+#pragma unroll
+    for (int d = 0; d < SIM_D; d++) stage(d, c + d);
+  }
+#pragma unroll
+  for (int d = 0; d < SIM_D - 1; d++)
+    if (c + d < nch) stage(d, c + d);
+  return 0.0f;
+}
+
+// k_sim_gate_up: block b owns units 32b .. 32b+31 (the routed units k*I + i, then the shared
+// expert's): rows 0-31 of sim_rows are their gate rows, 32-63 their up rows. Waves 0-4 route as k_dec_gate_up does
+// (each for itself). h = bf16(SwiGLU(bf16(g), bf16(u))); block 0 publishes the routing.
+__global__ void __launch_bounds__(SIM_THREADS) k_sim_gate_up(dsh_layer_t L, const float *x_in,
+                                                             const int *__restrict__ step, int stride,
+                                                             const float *partials, int np, int mode,
+                                                             dsh_layer_work_t wk) {
   __shared__ __attribute__((aligned(16))) float s_x[2048];
-  __shared__ int s_idx[4 * 64];
-  __shared__ float s_w[4 * 64];
+  __shared__ int s_idx[5 * 64];
+  __shared__ float s_w[5 * 64];
   __shared__ float s_red[4][64];
-  __shared__ float s_up[128];
   __shared__ float s_xsum;
+  __shared__ sim_smem S;
   const float *x = at_step(x_in, step, stride);
   const int H = L.H, I = L.I, K = L.K, SI = L.SI, KI = K * I;
   const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
-  for (int i = t; i < H; i += 320) s_x[i] = x[i];
-  if (wave < 4) {
+  const bool routed = (int)blockIdx.x * 32 < KI;  // the block has routed units
+  for (int i = t; i < H; i += SIM_THREADS) s_x[i] = x[i];
+  if (routed && wave < 4) {
     float pv[ROUTE_BATCH];
     route_load(partials, np, pv);
     route_reduce(np, L.E, pv, s_red, nullptr);
   }
   __syncthreads();  // s_x, s_red
-  const int u = blockIdx.x * 128 + (t & 127), part = (t >> 7) & 1;
-  const bool active = wave < 4 && u < KI + SI;
-  float dot = 0.0f;
+  if (routed && wave < 5) route_select(L.E, K, mode, s_idx + 64 * wave, s_w + 64 * wave, s_red);
+  const int *idx = s_idx + 64 * min(wave, 4);
+  int e = 0;  // of the row asked for last: the lane's own row in wave 4
+  // row r's number in its expert's (or the shared expert's) gate_up rows; units past the end repeat the last one
+  auto where = [&](int r, bool &sh) -> size_t {
+    const int u = min((int)blockIdx.x * 32 + (r & 31), KI + SI - 1), part = r >> 5;
+    sh = u >= KI;
+    if (sh) return (size_t)part * SI + (u - KI);
+    const int k = u / I;
+    e = idx[k];
+    return (size_t)max(e, 0) * 2 * I + (size_t)part * I + (u - k * I);
+  };
   float2 so = make_float2(0.0f, 0.0f);
-  int e = 0;
   if (wave == 4) {
-    if (lane == 0) {  // Σx, added in element order as the reference's loop does
-      float xs = 0.0f;
-      for (int i = 0; i < H; i += 4) {
-        const f32x4 v = *(const f32x4 *)(s_x + i);
-        xs += v[0];
-        xs += v[1];
-        xs += v[2];
-        xs += v[3];
-      }
-      s_xsum = xs;
-    }
-  } else {
-    route_select(L.E, K, mode, s_idx + 64 * wave, s_w + 64 * wave, s_red);
-    if (active) {
-      const int8_t *row;
-      if (u < KI) {
-        const int k = u / I, i = u - k * I;
-        e = s_idx[64 * wave + k];
-        const size_t r = (size_t)max(e, 0) * 2 * I + (size_t)part * I + i;
-        row = L.gu_q + r * H;
-        so = so_pair(L.gu_so, r);
-      } else {
-        const size_t r = (size_t)part * SI + (u - KI);
-        row = L.sgu_q + r * H;
-        so = so_pair(L.sgu_so, r);
-      }
-      float unused = 0.0f;
-      dot = dsh_row_chain<false>(row, s_x, H, unused);
-    }
+    bool sh;
+    const size_t r = where(lane, sh);
+    so = so_pair(sh ? L.sgu_so : L.gu_so, r);
   }
+  const float acc = sim_rows(S, s_x, H, [&](int r) {
+    bool sh;
+    const size_t at = where(r, sh);
+    return (sh ? L.sgu_q : L.gu_q) + at * H;
+  });
+  if (t == 64 * 5) s_xsum = acc;
   __syncthreads();  // s_xsum
-  float y = 0.0f;
-  if (active) {
-    y = dsh_bf16_round_half_up(__builtin_fmaf(so.x, dot, so.y * s_xsum));
-    if (part) s_up[t & 127] = y;
-  }
-  __syncthreads();  // s_up
-  if (active && !part) {
-    const float hv = dsh_bf16_round_half_up(dsh_swiglu(y, s_up[t]));
-    wk.h[u] = (u < KI && e < 0) ? 0.0f : hv;
+  if (wave == 4) {
+    const float y = dsh_bf16_round_half_up(__builtin_fmaf(so.x, acc, so.y * s_xsum));
+    const float up = __shfl_down(y, 32);
+    const int u = blockIdx.x * 32 + lane;
+    if (lane < 32 && u < KI + SI) wk.h[u] = u < KI && e < 0 ? 0.0f : dsh_bf16_round_half_up(dsh_swiglu(y, up));
   }
   if (blockIdx.x == 0 && wave == 0 && lane < K) {
     wk.idx[lane] = s_idx[lane];
@@ -635,50 +753,31 @@ __global__ void __launch_bounds__(320) k_sim_gate_up(dsh_layer_t L, const float 
   }
 }
 
-// k_sim_down: block (64-row tile, segment seg): lane r of wave 0 runs output row 64*tile + r of routed
-// slot seg (seg < K: expert idx[seg] on its I SwiGLU outputs) or of the shared expert (seg == K, on
-// its SI outputs); lane 0 of wave 1 sums h. e = bf16(fma(scale, dot, offset * Σh)) into eo[seg][row]
-// (0 for a DECODE slot left empty).
-__global__ void __launch_bounds__(128) k_sim_down(dsh_layer_t L, dsh_layer_work_t wk) {
+// k_sim_down: block (64-row tile, segment seg): the output rows of routed slot seg (seg < K: expert
+// idx[seg] on its I SwiGLU outputs) or of the shared expert (seg == K, on its SI outputs).
+// e = bf16(fma(scale, dot, offset * Σh)) into eo[seg][row] (0 for a DECODE slot left empty).
+__global__ void __launch_bounds__(SIM_THREADS) k_sim_down(dsh_layer_t L, dsh_layer_work_t wk) {
   __shared__ __attribute__((aligned(16))) float s_h[7 * 1024];
   __shared__ float s_hsum;
+  __shared__ sim_smem S;
   const int H = L.H, I = L.I, K = L.K, SI = L.SI;
-  const int seg = blockIdx.y, t = threadIdx.x, wave = t >> 6, lane = t & 63;
+  // the shared expert's blocks, whose chains are the longest, start first
+  const int seg = blockIdx.y ? (int)blockIdx.y - 1 : K, t = threadIdx.x, wave = t >> 6, lane = t & 63;
   const int n = seg < K ? I : SI;
   const float *h = wk.h + (seg < K ? seg * I : K * I);
-  for (int i = t; i < n; i += 128) s_h[i] = h[i];
+  if (wave >= 4)  // waves 0-3 go straight to their codes
+    for (int i = 4 * (t - 256); i < n; i += 512) *(f32x4 *)(s_h + i) = *(const f32x4 *)(h + i);
   const int e = seg < K ? wk.idx[seg] : 0;
-  __syncthreads();  // s_h
-  const int r = blockIdx.x * 64 + lane;
-  float dot = 0.0f;
+  const size_t r0 = (seg < K ? (size_t)max(e, 0) * H : 0) + blockIdx.x * 64;  // its rows, in the expert's or the shared ones
   float2 so = make_float2(0.0f, 0.0f);
-  if (wave == 0) {
-    const int8_t *row;
-    if (seg < K) {
-      const size_t rr = (size_t)max(e, 0) * H + r;
-      row = L.dn_q + rr * I;
-      so = so_pair(L.dn_so, rr);
-    } else {
-      row = L.sdn_q + (size_t)r * SI;
-      so = so_pair(L.sdn_so, r);
-    }
-    float unused = 0.0f;
-    dot = dsh_row_chain<false>(row, s_h, n, unused);
-  } else if (lane == 0) {
-    float hs = 0.0f;
-    for (int i = 0; i < n; i += 4) {
-      const f32x4 v = *(const f32x4 *)(s_h + i);
-      hs += v[0];
-      hs += v[1];
-      hs += v[2];
-      hs += v[3];
-    }
-    s_hsum = hs;
-  }
+  if (wave == 4) so = so_pair(seg < K ? L.dn_so : L.sdn_so, r0 + lane);
+  const int8_t *q = (seg < K ? L.dn_q : L.sdn_q) + r0 * n;
+  const float acc = sim_rows(S, s_h, n, [&](int r) { return q + (size_t)r * n; });
+  if (t == 64 * 5) s_hsum = acc;
   __syncthreads();  // s_hsum
-  if (wave == 0)
-    wk.eo[(size_t)seg * H + r] =
-        (seg < K && e < 0) ? 0.0f : dsh_bf16_round_half_up(__builtin_fmaf(so.x, dot, so.y * s_hsum));
+  if (wave == 4)
+    wk.eo[(size_t)seg * H + blockIdx.x * 64 + lane] =
+        (seg < K && e < 0) ? 0.0f : dsh_bf16_round_half_up(__builtin_fmaf(so.x, acc, so.y * s_hsum));
 }
 
 // k_sim_combine: R rows per 64-lane block, as k_dec_down's combine: out = Σ_k fma(w_k, e_k, out) in
@@ -1078,8 +1177,8 @@ hipError_t dsh_launch_dec_gate_up(const dsh_layer_t *L, const float *x_in, const
     return hipErrorInvalidValue;
   if (bf16sim) {  // every rounded value in the reference's order
     if (L->H > 2048 || L->H % 16) return hipErrorInvalidValue;
-    k_sim_gate_up<<<(L->K * L->I + L->SI + 127) / 128, 320, 0, s>>>(*L, x_in, step, stride, partials, np, route_mode,
-                                                                    *wk);
+    k_sim_gate_up<<<(L->K * L->I + L->SI + 31) / 32, SIM_THREADS, 0, s>>>(*L, x_in, step, stride, partials, np,
+                                                                          route_mode, *wk);
     return hipGetLastError();
   }
   const int blocks = dec_gate_up_blocks(L);
@@ -1101,7 +1200,7 @@ hipError_t dsh_launch_dec_down(const dsh_layer_t *L, const float *x_in, const in
                                const float *WrT_next, int E_next, float *partials_next, hipStream_t s) {
   if (bf16sim) {  // every rounded value in the reference's order, then the combine
     if (L->H % 64 || L->I % 16 || L->SI % 16 || L->SI > 7 * 1024 || !wk->eo) return hipErrorInvalidValue;
-    k_sim_down<<<dim3(L->H / 64, L->K + 1), 128, 0, s>>>(*L, *wk);
+    k_sim_down<<<dim3(L->H / 64, L->K + 1), SIM_THREADS, 0, s>>>(*L, *wk);
     if (dec_rows(L->H) == 8)
       k_sim_combine<8><<<L->H / 8, 64, 0, s>>>(*L, x_in, step, stride, x_out, residual, resid, *wk, WrT_next, E_next,
                                                 partials_next);

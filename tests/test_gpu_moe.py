@@ -90,6 +90,30 @@ def test_small_layer_vs_oracle(dev, B, mode, sim):
         L.ds_hip_layer_destroy(h)
 
 
+@pytest.mark.parametrize("hidden,inter,top_k", [(256, 16, 1), (256, 48, 7), (768, 144, 5), (256, 1024, 1), (2048, 272, 6)])
+def test_bf16sim_tile_edges(dev, B, hidden, inter, top_k):
+    """bf16 simulation where its kernels' tiles end: blocks of 32 units that reach over two slots, or from
+    the routed ones into the shared expert, or past the last unit; one, whole and partial chunks of 128
+    columns; the longest shared chain (7 x 1024). Bit-identical to the oracle."""
+    L = dev.load()
+    lay = B.make_moe_layer(83, hidden=hidden, inter=inter, n_experts=8, top_k=top_k, n_shared=8 - top_k)
+    h = upload_layer(dev, lay)
+    orl = lay.or_layer()
+    try:
+        dev.set_bf16sim(1)
+        for s in range(2):
+            x = B.normal_f32(hidden, 8300 + s)
+            out, idx, w = layer_forward(dev, h, x, dev.ROUTE_DECODE, K=top_k)
+            ro, ri, rw = np.empty(hidden, np.float32), np.empty(top_k, np.int32), np.empty(top_k, np.float32)
+            B.oracle().or_moe_layer_decode(ro, x, C.byref(orl), 0, 1, 1, ri, rw)
+            assert np.array_equal(idx, ri)
+            assert np.array_equal(bits(w), bits(rw))
+            assert np.array_equal(bits(out), bits(ro))
+    finally:
+        dev.set_bf16sim(0)
+        L.ds_hip_layer_destroy(h)
+
+
 @pytest.mark.parametrize("threads", [6, 5, 3, 16])
 def test_decode_routing_over_thread_chunks(dev, B, threads):
     """DECODE-mode router scores follow the reference's row chunking over its threads: with these
