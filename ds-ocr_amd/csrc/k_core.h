@@ -138,6 +138,10 @@ int dsh_pf_fused(void);
 /* 1 if a probe grid's blocks were dealt evenly over all 8 XCDs (runs the probe once, outside stream
  * capture): the fused prefill GEMM and the one-kernel layers' per-XCD verifiers rely on it. */
 int dsh_xcd_even(void);
+/* The fused launch's blocks per XCD for T tokens (-1: shape not supported), and the items of one expert that its
+ * plan puts into one queue unit at most: no queue has more tiles than blocks, whatever the routing. */
+int dsh_pf_queue_blocks(int H, int I, int SI, int E, int K, int T);
+int dsh_pf_unit_items(int T);
 /* 1 if a fused launch's bounded wait expired (its output is then not valid), 0 if not; synchronous. */
 int dsh_pf_wait_error(const void *ws, const dsh_layer_t *L, int T);
 /* out[T][H] = (residual ? X : 0) + MoE(X); ws: dsh_pf_workspace_bytes(L, T) device bytes. derr (may be

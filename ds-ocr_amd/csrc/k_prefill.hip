@@ -40,7 +40,7 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 #define PF_TB 8     // tokens per DECODE-mode scores block
 #define PF_PLAN_LDS 65536  // (token, slot) entries the plan kernel caches in LDS (a byte each)
 #define PF_NQ 8           // work queues of the fused GEMM kernel: one per XCD
-#define PF_UG 8           // items of one expert that share a queue, at most
+#define PF_UG 8           // items of one expert that share a queue unit, at most (pf_unit_items)
 #define PF_DN_TILE 0x80000000u  // tile word: down tile flag | item << 8 | n-tile
 
 // Work queues of the fused GEMM kernel (k_pf_moe), built by the plan kernel.
@@ -63,6 +63,13 @@ struct pf_queues {
 struct pf_hq {
   int8_t *r0, *r1, *s0, *s1;
 };
+
+// Items of one expert in a queue unit, at most: PF_UG, and no more than hold every token once. An expert has more
+// items than that only where a token lists it several times (CFG routing fills the empty slots of a token whose
+// scores are NaN or at the floor with expert 0). The launch bound (dsh_pf_queue_blocks) rests on this limit.
+__host__ __device__ constexpr int pf_unit_items(int T) {
+  return (T + PF_MT - 1) / PF_MT < PF_UG ? (T + PF_MT - 1) / PF_MT : PF_UG;
+}
 
 struct pf_item {
   int seg;   // expert 0..E-1, or E for the shared expert
@@ -530,7 +537,7 @@ __global__ void __launch_bounds__(1024) k_pf_plan(const int *__restrict__ idx, i
   __shared__ int run[16][64];
   __shared__ unsigned char cache[PF_PLAN_LDS];  // the entries' experts, 255: none
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int TK = T * K;
+  const int TK = T * K, unit = pf_unit_items(T);
   const bool cached = TK <= PF_PLAN_LDS;
   const int per = (TK + 15) / 16;
   const int lo = min(wave * per, TK), hi = min(lo + per, TK);
@@ -556,7 +563,7 @@ __global__ void __launch_bounds__(1024) k_pf_plan(const int *__restrict__ idx, i
 #pragma unroll
   for (int v = 0; v < 16; v++) c += cv[v];
   if (Q.enable && wave >= 1 && wave <= PF_UG) {  // wave v counts the queue units (below) of v items
-    const int nch = (c + PF_MT - 1) / PF_MT, ug = (nch + PF_UG - 1) / PF_UG, sz = ug ? nch / ug : 0, big = nch - sz * ug;
+    const int nch = (c + PF_MT - 1) / PF_MT, ug = (nch + unit - 1) / unit, sz = ug ? nch / ug : 0, big = nch - sz * ug;
     const int n = wave == sz ? ug - big : (wave == sz + 1 ? big : 0);
     int incl = n;
 #pragma unroll
@@ -616,7 +623,7 @@ __global__ void __launch_bounds__(1024) k_pf_plan(const int *__restrict__ idx, i
   if (threadIdx.x == 0) *Q.err = 0;
   __syncthreads();
   if (Q.enable) {
-    // Queue units are groups of up to PF_UG items of one expert (an expert's nch items in the fewest groups,
+    // Queue units are groups of up to pf_unit_items items of one expert (an expert's nch items in the fewest groups,
     // their sizes differing by at most one) and the single shared-expert items. A group's tiles run n-tile by n-tile,
     // its items side by side, on one XCD, so its weight rows come from HBM once and from that XCD's L2 for the other
     // items; so do the shared items of one queue. Units are ranked by cost (in 128-column weight stages), then by
@@ -686,7 +693,7 @@ __global__ void __launch_bounds__(1024) k_pf_plan(const int *__restrict__ idx, i
         int e = 0;  // the item's expert: the last whose first item is not past u (experts without items lie on it)
 #pragma unroll
         for (int d = 32; d; d >>= 1) e += s_ich[min(e + d, 63)] <= u && e + d < 64 ? d : 0;
-        const int nch = s_nch[e], i = u - s_ich[e], ug = (nch + PF_UG - 1) / PF_UG, sz = nch / ug, big = nch - sz * ug;
+        const int nch = s_nch[e], i = u - s_ich[e], ug = (nch + unit - 1) / unit, sz = nch / ug, big = nch - sz * ug;
         const int nb = big * (sz + 1);  // the expert's larger groups come first
         z = i < nb ? sz + 1 : sz;
         const int g = i < nb ? i / (sz + 1) : (i - nb) / sz;
@@ -1525,6 +1532,20 @@ size_t pf_queue_cap(const dsh_layer_t *L, int T) {
   return r * (L->I / pf_tile_t::GU) + sh * (L->SI / pf_tile_t::GU) + (r + sh) * (L->H / pf_tile_t::DN);
 }
 
+// Blocks per XCD of the fused launch, at least the tiles of the longest queue: its cost is at most the mean and the
+// costliest unit (the units are dealt in snake order by cost; a unit is one shared item or at most pf_unit_items
+// items of one expert), and a tile costs at least the smaller of the kinds' means.
+long pf_queue_blocks(const dsh_layer_t *L, int T) {
+  const int nr = pf_max_routed_items(L, T), ns = pf_shared_items(T);
+  const int ngu_r = L->I / pf_tile_t::GU, ngu_s = L->SI / pf_tile_t::GU, ndn = L->H / pf_tile_t::DN;
+  const long cost_r = (long)ngu_r * (L->H / PF_KS) + (long)ndn * (L->I / PF_KS);
+  const long cost_s = (long)ngu_s * (L->H / PF_KS) + (long)ndn * (L->SI / PF_KS);
+  const long unit = max(cost_s, pf_unit_items(T) * cost_r);
+  const long longest = (nr * cost_r + ns * cost_s + PF_NQ - 1) / PF_NQ + unit;
+  const long tiles = max(longest * (ngu_r + ndn) / cost_r, longest * (ngu_s + ndn) / cost_s) + 1;
+  return min(tiles, (long)pf_queue_cap(L, T));
+}
+
 int g_pf_xcd_min = 0;  // fewest blocks any XCD received out of a probe grid of PF_PROBE blocks
 int g_pf_auto = -1;   // -1 unchecked, 1 the grid's blocks cover all PF_NQ XCDs, 0 not
 int g_pf_fused = -1;  // path in use
@@ -1583,6 +1604,14 @@ int dsh_pf_supported(const dsh_layer_t *L) {
   if (L->I > PF_EU * PF_NT_MAX || L->SI > PF_EU * PF_NT_MAX) return 0;  // down: exponent table per row
   return 1;
 }
+
+int dsh_pf_queue_blocks(int H, int I, int SI, int E, int K, int T) {
+  dsh_layer_t L = {};
+  L.H = H, L.I = I, L.SI = SI, L.E = E, L.K = K;
+  return dsh_pf_supported(&L) && T > 0 ? (int)pf_queue_blocks(&L, T) : -1;
+}
+
+int dsh_pf_unit_items(int T) { return pf_unit_items(T); }
 
 size_t dsh_pf_workspace_bytes(const dsh_layer_t *L, int T) { return pf_carve(L, T, NULL, NULL); }
 
@@ -1708,16 +1737,7 @@ hipError_t dsh_launch_prefill(const dsh_layer_t *L, const float *X, int T, int r
   k_pf_plan<<<1, 1024, 0, s>>>(w.idx, T, K, E, L->I / pf_tile_t::GU, H / pf_tile_t::DN, w.seg_off, w.items, w.counts,
                                w.tiles_gu, w.tiles_dn, w.pair_tok, w.pos_of, Q);
   if (fused) {
-    // blocks per XCD >= tiles of the longest queue, whose cost is at most the mean and the costliest unit (dealt in
-    // snake order by cost); a tile costs at least the smaller of the kinds' means
-    const int nr_max = pf_max_routed_items(L, T), ns = pf_shared_items(T);
-    const int tr = Q.ngu_r + Q.ndn, ts = Q.ngu_s + Q.ndn;
-    const long cost_r = (long)Q.ngu_r * Q.nk_gu + (long)Q.ndn * Q.nk_dr;
-    const long cost_s = (long)Q.ngu_s * Q.nk_gu + (long)Q.ndn * Q.nk_ds;
-    const long unit = max(cost_s, min((long)PF_UG, (long)ns) * cost_r);
-    const long longest = (nr_max * cost_r + ns * cost_s + PF_NQ - 1) / PF_NQ + unit;
-    const long tiles = max(longest * tr / cost_r, longest * ts / cost_s) + 1;
-    const int blocks = (int)min((long)PF_NQ * tiles, (long)PF_NQ * Q.cap);
+    const int blocks = (int)(PF_NQ * pf_queue_blocks(L, T));
     k_pf_moe<<<blocks, 256, 0, s>>>(*L, w.items, Q, w.X0, w.X1, w.xsc, w.xsum, w.pair_tok, bf16sim, w.hq, w.hpr,
                                     w.hps, w.hmr, w.hms, w.Y, w.Ysh);
   } else {

@@ -442,6 +442,34 @@ def test_prefill_nonfinite_tokens(dev, B, mode, path):
         L.ds_hip_layer_destroy(h)
 
 
+@pytest.mark.parametrize("E,H,I,T,bad", [(16, 256, 128, 66, 54), (16, 256, 128, 128, 64), (16, 256, 128, 130, 122),
+                                         (64, 256, 128, 128, 64), (64, 1280, 896, 128, 64)])
+def test_prefill_mostly_nan_tokens(dev, B, path, E, H, I, T, bad):
+    """CFG routing lists expert 0 six times for a token whose scores are all NaN, so with many such tokens expert 0
+    has more items than a prompt of ordinary tokens can give it, and one work queue most of the tiles. Every tile
+    must run all the same: the ordinary tokens' outputs, indices and weights are bit-identical to those of a
+    call in which every token is ordinary. A call on other tokens comes between the two, so that a row left from
+    the first one does not pass for a computed one."""
+    L = dev.load()
+    h = make_device_layer(dev, 68, H=H, I=I, E=E, SI=2 * I)[0]
+    try:
+        X = np.stack([B.normal_f32(H, 6800 + t) for t in range(T)])
+        ok = gpu_prefill(dev, h, X, 1, residual=1)
+        gpu_prefill(dev, h, X[::-1].copy() * np.float32(3), 1, residual=1)
+        Xb = X.copy()
+        nan = np.sort(np.random.default_rng(68).permutation(T)[:bad])
+        Xb[nan, nan % H] = np.nan
+        got = gpu_prefill(dev, h, Xb, 1, residual=1)
+        good = np.setdiff1d(np.arange(T), nan)
+        assert np.array_equal(got[1][nan], np.zeros((bad, 6), np.int32))
+        for a, b in zip(got, ok):
+            differ = (a.view(np.uint32) != b.view(np.uint32)).any(axis=1)
+            assert not differ[good].any(), np.flatnonzero(differ[good])
+        assert np.isnan(got[0][nan]).all()
+    finally:
+        L.ds_hip_layer_destroy(h)
+
+
 @pytest.mark.parametrize("mode", [0, 1])
 def test_prefill_zero_h_tile(dev, B, mode, path):
     """The gate rows of units 0-127 of every expert are zero, so each row's h is zero over its first
