@@ -864,12 +864,14 @@ __global__ void __launch_bounds__(256) k_sum_pairs_f64(const double *__restrict_
 // ============================================================================ f32 GEMM, bf16 weights
 // Y[M,N] = X[M,K] * W[N,K]^T with W widened from bf16 (ds_linear_nobias_bf16, seq_len > 1: the
 // reference converts W to f32 and calls sgemm, ds_kernels.c:917-927), on the bf16 MFMA: x is split into three bf16
-// numbers of 8 bits each, x = x1 + x2 + x3 exactly, so every product w x_i is exact in f32 and only the sums round, 32
-// columns to an MFMA step instead of one to a fused multiply-add (error against f64 at K = 1280: 2.1e-7 relative,
+// numbers of 8 bits each, x = x1 + x2 + x3 exactly for |x| >= 2^-103 (below, the parts run into bf16's subnormal grid,
+// and from 2^-110 on lose bits), so every product w x_i is exact in f32 and only the sums round, 32 columns to an MFMA step instead of one to a fused multiply-add (error against f64 at K = 1280: 2.1e-7 relative,
 // 6.4e-7 for the chain of fused multiply-adds). A block of 4 waves takes 64 x 64 of Y, a wave 32 x 32; K runs in
 // stages of 64 columns, split on their way into LDS (rows of 72 elements: 16-byte reads of 16 rows spread over
 // all banks), the next stage on its way in registers. At 662 x 1280 x 1280 (220 blocks) bound by the 20 stages'
 // latency: 28.7 us, 227 us for scalar f32 tiles. VEC: K % 8 == 0 (16-byte loads of both operands' rows).
+// A tile with a smaller x other than zero in its rows goes through gb_tile_fma, 8 times as slow; looking for one costs
+// 0.9 us of a kernel at K = 1280 (two instructions per element, one more reduction over the block).
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef unsigned short u16x8 __attribute__((ext_vector_type(8)));
 #define GB_KS 64
@@ -885,6 +887,44 @@ __device__ __forceinline__ void gb_split(float x, unsigned short &a, unsigned sh
   b = (unsigned short)(fin ? ur >> 16 : 0u);
   c = (unsigned short)(fin ? __float_as_uint(q) >> 16 : 0u);
 }
+#define GB_MIN 0x0C000000u  // 2^-103
+// A 64 x 64 tile of Y by chains of fused multiply-adds in column order, whatever the size of x: 16 columns of both
+// operands at a time in LDS (lds: 2 x 16 x 65 floats), 4 x 4 outputs per thread.
+__device__ __forceinline__ void gb_tile_fma(const float *X, const uint16_t *W, float *Y, int M, int K, int N, int m0,
+                                            int n0, float *lds) {
+  float(*xs)[65] = (float(*)[65])lds, (*ws)[65] = xs + 16;
+  const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
+  float acc[4][4] = {};
+  for (int k0 = 0; k0 < K; k0 += 16) {
+    for (int i = threadIdx.x; i < 16 * 64; i += 256) {
+      const int kk = i & 15, rr = i >> 4, m = m0 + rr, n = n0 + rr, k = k0 + kk;
+      xs[kk][rr] = m < M && k < K ? X[(size_t)m * K + k] : 0.0f;
+      ws[kk][rr] = n < N && k < K ? dsh_bf16_to_f32(W[(size_t)n * K + k]) : 0.0f;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int kk = 0; kk < 16; kk++) {
+      float a[4], b[4];
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        a[i] = xs[kk][4 * ty + i];
+        b[i] = ws[kk][4 * tx + i];
+      }
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) acc[i][j] = __builtin_fmaf(a[i], b[j], acc[i][j]);
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int i = 0; i < 4; i++)
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const int m = m0 + 4 * ty + i, n = n0 + 4 * tx + j;
+      if (m < M && n < N) Y[(size_t)m * N + n] = acc[i][j];
+    }
+}
 template <bool VEC>
 __global__ void __launch_bounds__(256) k_gemm_bf16w(const float *__restrict__ X, const uint16_t *__restrict__ W,
                                                     float *__restrict__ Y, int M, int K, int N) {
@@ -898,6 +938,7 @@ __global__ void __launch_bounds__(256) k_gemm_bf16w(const float *__restrict__ X,
   const uint16_t *wrow = W + (size_t)min(n0 + cr, N - 1) * K;
   float xr[16];
   unsigned short wr[16];
+  uint32_t least = ~0u;  // of the thread's x so far but zeros: 2 * (the least magnitude's bits) - 1
   auto load = [&](int k0) {
     const int k = k0 + cc;
     if (VEC) {
@@ -931,6 +972,7 @@ __global__ void __launch_bounds__(256) k_gemm_bf16w(const float *__restrict__ X,
       for (int i = 0; i < 8; i++) {
         unsigned short a, c, d;
         gb_split(xr[8 * h + i], a, c, d);
+        least = min(least, 2u * __float_as_uint(xr[8 * h + i]) - 1u);
         p[0][i] = a;
         p[1][i] = c;
         p[2][i] = d;
@@ -968,6 +1010,10 @@ __global__ void __launch_bounds__(256) k_gemm_bf16w(const float *__restrict__ X,
         }
     }
     if (k + 1 < nk) store(b ^ 1);  // the other buffer: every wave was done with it before the last barrier
+  }
+  if (__syncthreads_or(least < 2u * GB_MIN - 1u)) {
+    gb_tile_fma(X, W, Y, M, K, N, m0, n0, (float *)s_x);
+    return;
   }
 #pragma unroll
   for (int i = 0; i < 2; i++)

@@ -360,3 +360,33 @@ def test_linear_bf16_batched_shapes(dev, B, M, K, N, scale):
     got = Y.reshape(M, N)
     assert np.array_equal(np.isnan(got), np.isnan(ref))
     assert np.array_equal(np.isinf(got), np.isinf(ref)) and np.array_equal(got[np.isinf(got)], ref[np.isinf(got)])
+
+
+@pytest.mark.parametrize("K", [7, 64, 1280])
+@pytest.mark.parametrize("exp2", [-100, -104, -109, -110, -111, -120, -126, -135, -145])
+def test_linear_bf16_batched_small_x(dev, B, K, exp2):
+    """x down to f32's smallest subnormals, in every row and as single elements among ordinary ones whose weights are
+    zero. A product or sum rounds by 2^-24 of itself or, where it is subnormal, by 2^-150: at most K + 3 roundings
+    on any partial sum. An infinite weight gives an infinity also with a subnormal x."""
+    L = dev.load()
+    M, N = 70, 66
+    X = (B.normal_f32(M * K, 430 + K) * np.float32(2.0 ** exp2)).reshape(M, K)
+    X[1:64:2] = B.normal_f32(32 * K, 431 + K).reshape(32, K)  # the second tile of rows has small x only
+    W = B.normal_bf16(N * K, 432 + K, 0.05).reshape(N, K)
+    X[5, K // 2] = np.float32(1.7 * 2.0 ** exp2)
+    W[3] = 0
+    W[3, K // 2] = 0x3F80  # output [5, 3] is that element
+    Y = np.empty((M, N), np.float32)
+    L.ds_linear_nobias_bf16(Y.reshape(-1), X.reshape(-1), W.reshape(-1), M, K, N)
+    W64 = B.bf16_to_f32(W.reshape(-1)).reshape(N, K).astype(np.float64)
+    ref, size = X.astype(np.float64) @ W64.T, np.abs(X).astype(np.float64) @ np.abs(W64.T)
+    assert Y[5, 3] == X[5, K // 2]
+    assert np.all(np.abs(Y - ref) <= (K + 3) * (2.0 ** -24 * size + 2.0 ** -150))
+    W2 = W.copy()
+    W2[2, 0] = 0x7F80
+    L.ds_linear_nobias_bf16(Y.reshape(-1), X.reshape(-1), W2.reshape(-1), M, K, N)
+    for w in (W, W2):
+        L.ds_hip_weights_changed(w.ctypes.data)
+    with np.errstate(invalid="ignore"):
+        ref = X[:, 0].astype(np.float64) * np.inf
+    assert np.array_equal(np.isnan(Y[:, 2]), np.isnan(ref)) and np.array_equal(Y[~np.isnan(ref), 2], ref[~np.isnan(ref)])
