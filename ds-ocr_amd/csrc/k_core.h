@@ -142,6 +142,10 @@ int dsh_xcd_even(void);
  * plan puts into one queue unit at most: no queue has more tiles than blocks, whatever the routing. */
 int dsh_pf_queue_blocks(int H, int I, int SI, int E, int K, int T);
 int dsh_pf_unit_items(int T);
+/* The kernel that computes a prompt's DECODE router scores: one for rows on any path of the reference's order, one with
+ * the rows in registers, one on the f32 MFMA. All give the same bits. */
+enum { DSH_PF_SCORES_ANY, DSH_PF_SCORES_REGS, DSH_PF_SCORES_MFMA };
+int dsh_pf_scores_kind(int H, int E, int T, int nthreads);
 /* 1 if a fused launch's bounded wait expired (its output is then not valid), 0 if not; synchronous. */
 int dsh_pf_wait_error(const void *ws, const dsh_layer_t *L, int T);
 /* out[T][H] = (residual ? X : 0) + MoE(X); ws: dsh_pf_workspace_bytes(L, T) device bytes. derr (may be

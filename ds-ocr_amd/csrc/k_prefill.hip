@@ -1546,6 +1546,23 @@ long pf_queue_blocks(const dsh_layer_t *L, int T) {
   return min(tiles, (long)pf_queue_cap(L, T));
 }
 
+// The kernel of the DECODE scores (H a multiple of 256). k_pf_scores_bf16 takes any row path; the others need every row
+// on a group path (the chunks of the reference's threads all have an even length). The one with the rows in
+// registers (H <= 1280) makes a pass per token of its block (256 blocks up to 256 tokens, then tpb tokens each), the
+// MFMA one a pass over the columns whatever the tokens. Each line lies where the two sides cross, in us with 64 experts:
+//   H 256,  tpb 8 / 9: 7.3 and 8.1 in registers, 8.0 MFMA;   H 512 and 768, tpb 7 / 8: 9.5, 10.4 and 10.0; 11.4, 12.5 and 12.0
+//   H 1024, tpb 4 / 5: 13.7, 16.4 and 14.0;                  H 1280, tpb 3 / 4: 13.7, 16.8 and 16.0 (3001 tokens: 43.4, 16.6)
+//   H > 1280 (no rows in registers), 1 / 2 / 3 tokens: H 1536 7.0, 12.6, 18.1 per token from L2 and 15.9, 16.5, 17.0 MFMA;
+//   H 2048 8.6, 15.9, 22.9 and 19.8, 20.5, 21.1
+int pf_scores_kind(int H, int E, int T, int nthreads) {
+  const int chunk = dsh_chunk_len(E, nthreads);
+  for (int s0 = 0; s0 < E; s0 += chunk)
+    if (min(chunk, E - s0) % 2) return DSH_PF_SCORES_ANY;
+  if (H > 1280) return T <= 2 ? DSH_PF_SCORES_ANY : DSH_PF_SCORES_MFMA;
+  const int tpb = (T + 255) / 256, most = H <= 256 ? 8 : H <= 768 ? 7 : H <= 1024 ? 4 : 3;
+  return tpb <= most ? DSH_PF_SCORES_REGS : DSH_PF_SCORES_MFMA;
+}
+
 int g_pf_xcd_min = 0;  // fewest blocks any XCD received out of a probe grid of PF_PROBE blocks
 int g_pf_auto = -1;   // -1 unchecked, 1 the grid's blocks cover all PF_NQ XCDs, 0 not
 int g_pf_fused = -1;  // path in use
@@ -1610,6 +1627,8 @@ int dsh_pf_queue_blocks(int H, int I, int SI, int E, int K, int T) {
   L.H = H, L.I = I, L.SI = SI, L.E = E, L.K = K;
   return dsh_pf_supported(&L) && T > 0 ? (int)pf_queue_blocks(&L, T) : -1;
 }
+
+int dsh_pf_scores_kind(int H, int E, int T, int nthreads) { return pf_scores_kind(H, E, T, nthreads); }
 
 int dsh_pf_unit_items(int T) { return pf_unit_items(T); }
 
@@ -1706,24 +1725,21 @@ hipError_t dsh_launch_prefill(const dsh_layer_t *L, const float *X, int T, int r
       k_pf_route_cfg<false><<<(T + 3) / 4, 256, 0, s>>>(L->router_f32_t, X, T, H, E, K, w.X0, w.X1, w.xsc, w.xsum,
                                                          w.idx, w.w, idx_out, w_out);
   } else {
-    // every row on a group path: the chunks of the reference's threads all have an even length
-    const int chunk = dsh_chunk_len(E, nthreads);
-    bool grouped = true;
-    for (int s0 = 0; s0 < E; s0 += chunk) grouped = grouped && (min(chunk, E - s0) % 2 == 0);
     const int tpb = (T + 255) / 256, nbr = (T + tpb - 1) / tpb;
 #define PFR(N)                                                                                                      \
   case N:                                                                                                           \
     k_pf_scores_bf16r<N><<<nbr, 256, 0, s>>>(L->router_bf16, X, T, E, tpb, w.ps);                                 \
     break;
-    // the MFMA kernel takes one pass whatever the tokens (up to 8192: two blocks per CU; 18.5 us at 3001), the one with
-    // the rows in registers a pass per token of a block (7 us with one, 14.5 with three, 46.5 with twelve)
-    if (grouped && H % 256 == 0 && (tpb > 3 || H > 1280)) {
-      k_pf_scores_mfma<<<(T + PF_SM_T - 1) / PF_SM_T, 256, 0, s>>>(L->router_bf16, X, T, H, E, w.ps);
-    } else if (grouped && H % 256 == 0) {
-      switch (H / 32) { PFR(8) PFR(16) PFR(24) PFR(32) PFR(40) }
-    } else {
-      k_pf_scores_bf16<<<(T + PF_TB - 1) / PF_TB, 256, (size_t)PF_TB * H * sizeof(float), s>>>(
-          L->router_bf16, X, T, H, E, nthreads, w.ps);
+    switch (pf_scores_kind(H, E, T, nthreads)) {
+      case DSH_PF_SCORES_MFMA:
+        k_pf_scores_mfma<<<(T + PF_SM_T - 1) / PF_SM_T, 256, 0, s>>>(L->router_bf16, X, T, H, E, w.ps);
+        break;
+      case DSH_PF_SCORES_REGS:
+        switch (H / 32) { PFR(8) PFR(16) PFR(24) PFR(32) PFR(40) }
+        break;
+      default:
+        k_pf_scores_bf16<<<(T + PF_TB - 1) / PF_TB, 256, (size_t)PF_TB * H * sizeof(float), s>>>(
+            L->router_bf16, X, T, H, E, nthreads, w.ps);
     }
 #undef PFR
     k_pf_select_dec<<<(T + 3) / 4, 256, 0, s>>>(X, T, H, E, K, w.ps, w.X0, w.X1, w.xsc, w.xsum, w.idx, w.w, idx_out,

@@ -400,6 +400,21 @@ def test_prefill_hidden_sizes(dev, B, mode, hidden):
         L.ds_hip_layer_destroy(h)
 
 
+@pytest.mark.parametrize("hidden,T", [(1536, 2), (1536, 3), (2048, 1), (2048, 2), (2048, 3), (256, 2048), (256, 2049),
+                                      (768, 1792), (768, 1793), (1024, 1024), (1024, 1025)])
+def test_prefill_decode_scores_kernel_edges(dev, B, hidden, T):
+    """DECODE routing on both sides of each line between two scores kernels: indices and weights bit for bit."""
+    L = dev.load()
+    lay = B.make_moe_layer(73, hidden=hidden, inter=128, n_experts=16)
+    h = upload_layer(dev, lay)
+    try:
+        X = B.normal_f32(T * hidden, 7300 + T).reshape(T, hidden)
+        out, idx, w = gpu_prefill(dev, h, X, 0)
+        check_routing(B, lay, X, idx, w, 0)
+    finally:
+        L.ds_hip_layer_destroy(h)
+
+
 @pytest.mark.parametrize("mode", [0, 1])
 def test_prefill_nonfinite_tokens(dev, B, mode, path):
     """Tokens with a +inf, a NaN or a -inf coordinate among ordinary ones. Each token's row is
