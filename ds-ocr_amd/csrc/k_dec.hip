@@ -580,7 +580,8 @@ __device__ __forceinline__ f32x4 sim_codes(unsigned w) {
 }
 // 16 steps: acc = fma(q_e, x_e, acc), or acc + x_e with SUM; lane e of every 16 holds x_e in v. In assembly, as the
 // compiler puts s_nop 1 between the steps: only a DPP operand (v, from LDS) must not come from the two instructions
-// before, which the one s_nop here covers.
+// before, which the one s_nop here covers. acc is written before the last operand is read: +&v keeps the operands out of
+// its register.
 #define SIM_BC(e) " row_newbcast:" #e " row_mask:0xf bank_mask:0xf\n"
 #define SIM_FMA(e, q) "v_fmac_f32_dpp %0, %1, %" #q SIM_BC(e)
 #define SIM_ADD(e) "v_add_f32_dpp %0, %1, %0" SIM_BC(e)
@@ -589,13 +590,13 @@ __device__ __forceinline__ float sim_steps(float acc, const f32x4 *q, float v) {
   if (SUM)
     asm volatile("s_nop 1\n" SIM_ADD(0) SIM_ADD(1) SIM_ADD(2) SIM_ADD(3) SIM_ADD(4) SIM_ADD(5) SIM_ADD(6) SIM_ADD(7)
                      SIM_ADD(8) SIM_ADD(9) SIM_ADD(10) SIM_ADD(11) SIM_ADD(12) SIM_ADD(13) SIM_ADD(14) SIM_ADD(15)
-                 : "+v"(acc)
+                 : "+&v"(acc)
                  : "v"(v));
   else
     asm volatile("s_nop 1\n" SIM_FMA(0, 2) SIM_FMA(1, 3) SIM_FMA(2, 4) SIM_FMA(3, 5) SIM_FMA(4, 6) SIM_FMA(5, 7)
                      SIM_FMA(6, 8) SIM_FMA(7, 9) SIM_FMA(8, 10) SIM_FMA(9, 11) SIM_FMA(10, 12) SIM_FMA(11, 13)
                          SIM_FMA(12, 14) SIM_FMA(13, 15) SIM_FMA(14, 16) SIM_FMA(15, 17)
-                 : "+v"(acc)
+                 : "+&v"(acc)
                  : "v"(v), "v"(q[0][0]), "v"(q[0][1]), "v"(q[0][2]), "v"(q[0][3]), "v"(q[1][0]), "v"(q[1][1]),
                    "v"(q[1][2]), "v"(q[1][3]), "v"(q[2][0]), "v"(q[2][1]), "v"(q[2][2]), "v"(q[2][3]), "v"(q[3][0]),
                    "v"(q[3][1]), "v"(q[3][2]), "v"(q[3][3]));
