@@ -770,6 +770,7 @@ __device__ __forceinline__ bool pf_tile(const int *counts, const int *tiles, int
 // codes. K runs in stages of PF_KS = 128 columns (one 128-byte line of each weight row), two
 // 64-column MFMA slices each; pf_mainloop_i8 below gives the details.
 #define PF_KS 128
+static_assert(PF_EU == PF_KS, "the down main loop takes one exponent of h per row and stage");
 #ifndef PF_OCC
 #define PF_OCC 2  // GEMM blocks per CU the register budget is sized for
 #endif

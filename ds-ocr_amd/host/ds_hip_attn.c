@@ -8,6 +8,13 @@
 #include "ds_hip.h"
 #include "dsr.h"
 
+/* What the kernels' arrays and half-wave scans hold for the longest cache: four 64-position chunks per part, a part per
+ * lane of half a wave, and the score maxima that a wave reads. */
+_Static_assert(DS_HIP_ATTN_MAX_SEQ <= 4 * 64 * DSH_ATTN_PARTS, "k_attn_av: four chunks per block");
+_Static_assert(DSH_ATTN_PARTS <= 32, "k_attn_oproj: half a wave per head");
+_Static_assert(DSH_ATTN_CM(DS_HIP_ATTN_MAX_SEQ) <= DSH_ATTN_CM_MAX && DSH_ATTN_CM_MAX % 64 == 0,
+               "k_attn_av: maxima read by a wave");
+
 struct ds_hip_attn {
   dsh_attn_t d;
   void *arena;
