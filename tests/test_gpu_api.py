@@ -338,7 +338,8 @@ def test_linear_bf16_batched(dev, B):
                                    (662, 1280, 96)])
 @pytest.mark.parametrize("scale", [1.0, 1e-30, 1e30])
 def test_linear_bf16_batched_shapes(dev, B, M, K, N, scale):
-    """Tile edges, odd K (rows that are not aligned) and magnitudes near both ends of f32. Every product is exact, so an
+    """Tile edges, odd K (rows that are not aligned) and magnitudes from 1e-30 to 1e30 (smaller ones:
+    test_linear_bf16_batched_small_x). Every product is exact, so an
     element differs from f64 by the roundings of its sum: at most K + 3 of them (2^-24 each) on any partial sum,
     which is at most the sum of |x w|. Infinities and NaN: the same classes as f64 gives."""
     L = dev.load()

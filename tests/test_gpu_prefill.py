@@ -90,7 +90,7 @@ def test_prefill_small_layer(dev, B, mode, T, path):
 def test_prefill_uneven_experts(dev, B, mode, T):
     """Tokens that lean the same way: a few experts get nearly all of them, the others none or a few. Item sizes around
     the 16-, 32- and 64-row tiles, experts whose items fill several queue groups (more than eight items), experts
-    without items, and (T > 768, DECODE) the scores on the f32 MFMA. TOL covers the 16-bit activation grid, which
+    without items. TOL covers the 16-bit activation grid, which
     does not depend on T."""
     L = dev.load()
     lay = B.make_moe_layer(65, hidden=256, inter=128, n_experts=16)
@@ -381,7 +381,7 @@ def test_prefill_config3_decode_routing(dev, B):
 def test_prefill_hidden_sizes(dev, B, mode, hidden):
     """The routing kernels at other hidden sizes: CFG scores in ds_linear's order (the router staged
     in 128-row chunks: 4, 8 and 16 of them) and DECODE scores with the router columns in registers
-    (512, 1024) or streamed per token (2048); indices bit for bit, weights as check_routing asks;
+    (512, 1024) or on the f32 MFMA (2048); indices bit for bit, weights as check_routing asks;
     the block output within the tolerance of the f64 brute force."""
     L = dev.load()
     lay = B.make_moe_layer(68 + hidden // 512, hidden=hidden, inter=128, n_experts=16)
@@ -412,6 +412,103 @@ def test_prefill_decode_scores_kernel_edges(dev, B, hidden, T):
         out, idx, w = gpu_prefill(dev, h, X, 0)
         check_routing(B, lay, X, idx, w, 0)
     finally:
+        L.ds_hip_layer_destroy(h)
+
+
+@pytest.mark.parametrize("hidden,E,T", [(1280, 64, 777), (512, 40, 1801), (2048, 64, 5), (1536, 16, 33), (256, 64, 2305)])
+def test_prefill_decode_scores_mfma(dev, B, hidden, E, T):
+    """DECODE scores on the f32 MFMA: all 64 experts of the instruction's four blocks, fewer than 64, and tokens that
+    fill no whole block of 16; indices and weights bit for bit, on tokens with a leaning of their own for some expert, so
+    that every expert is chosen."""
+    L = dev.load()
+    h, rf, rb = make_device_layer(dev, 74, H=hidden, I=128, E=E, SI=256)
+    old = L.ds_get_threads()
+    try:
+        L.ds_set_threads(1)
+        assert L.dsh_pf_scores_kind(hidden, E, T, 1) == 2
+        lay = export_layer(dev, B, h, rf, rb, H=hidden, I=128, E=E, SI=256)
+        R = B.bf16_to_f32(lay.router_bf16).reshape(E, hidden)
+        X = B.normal_f32(T * hidden, 7400 + T).reshape(T, hidden) + 2 * R[np.arange(T) % E] / R.std()
+        X = X.astype(np.float32) * np.float32(0.2)
+        out, idx, w = gpu_prefill(dev, h, X, 0)
+        check_routing(B, lay, X, idx, w, 0)
+        assert len(np.unique(idx)) == E or T < E
+    finally:
+        L.ds_set_threads(old)
+        L.ds_hip_layer_destroy(h)
+
+
+def test_prefill_decode_scores_mfma_nonfinite_tokens(dev, B):
+    """Tokens with infinities and NaN through the f32 MFMA scores: their routing is the oracle's on the same token (the
+    same slots empty, the same weights or NaN), and the tokens beside them, which share their blocks, keep theirs."""
+    L = dev.load()
+    T, H, E = 37, 1536, 64
+    h, rf, rb = make_device_layer(dev, 75, H=H, I=128, E=E, SI=256)
+    old = L.ds_get_threads()
+    try:
+        L.ds_set_threads(1)
+        assert L.dsh_pf_scores_kind(H, E, T, 1) == 2
+        lay = export_layer(dev, B, h, rf, rb, H=H, I=128, E=E, SI=256)
+        X = B.normal_f32(T * H, 7500).reshape(T, H) * np.float32(0.3)
+        for t, c, v in ((0, 3, np.inf), (5, 700, np.nan), (17, 1535, -np.inf), (31, 64, 3e38), (36, 9, np.nan)):
+            X[t, c] = v
+        out, idx, w = gpu_prefill(dev, h, X, 0)
+        for t in range(T):
+            sc = np.empty(E, np.float32)
+            B.oracle().or_bf16_matvec_avx512(sc, X[t], lay.router_bf16, H, E, 1)
+            ri, rw = np.empty(6, np.int32), np.empty(6, np.float32)
+            B.oracle().or_softmax_topk_decode(ri, rw, sc, E, 6)
+            assert np.array_equal(ri, idx[t]), (t, ri, idx[t])
+            nan = np.isnan(rw)
+            assert np.array_equal(nan, np.isnan(w[t])) and np.array_equal(rw[~nan].view(np.uint32),
+                                                                          w[t][~nan].view(np.uint32)), t
+    finally:
+        L.ds_set_threads(old)
+        L.ds_hip_layer_destroy(h)
+
+
+@pytest.mark.parametrize("T", [10922, 10923])
+def test_prefill_plan_past_its_lds(dev, B, path, T):
+    """The most (token, slot) pairs that the plan keeps in LDS (65532 of 65536) and the first prompt past that, which
+    reads them again: routing of every token, the output of 32 of them."""
+    L = dev.load()
+    H = 256
+    lay = B.make_moe_layer(76, hidden=H, inter=128, n_experts=16)
+    h = upload_layer(dev, lay)
+    try:
+        X = B.normal_f32(T * H, 7600).reshape(T, H)
+        out, idx, w = gpu_prefill(dev, h, X, 1)
+        check_routing(B, lay, X, idx, w, 1)
+        rows = np.linspace(0, T - 1, 32).astype(int)
+        ref = np.empty((len(rows), H), np.float64)
+        B.oracle().or_prefill_moe_f64(ref, np.ascontiguousarray(X[rows]), len(rows), C.byref(lay.or_layer()),
+                                     np.ascontiguousarray(idx[rows]), np.ascontiguousarray(w[rows]))
+        assert rel_err(out[rows], ref) < TOL
+    finally:
+        L.ds_hip_layer_destroy(h)
+
+
+@pytest.mark.parametrize("T", [7, 40, 130])
+def test_prefill_bf16sim(dev, B, path, T):
+    """bf16 simulation: gate and up, h and every expert's output rounded to bf16 (2^-9 relative each, so at most 4 of them
+    on the way to an output, besides TOL), over items of 16, 32 and 64 rows; without it the same call is closer."""
+    L = dev.load()
+    H = 256
+    lay = B.make_moe_layer(77, hidden=H, inter=128, n_experts=16)
+    h = upload_layer(dev, lay)
+    try:
+        X = B.normal_f32(T * H, 7700 + T).reshape(T, H)
+        err = []
+        for sim in (1, 0):
+            dev.set_bf16sim(sim)
+            out, idx, w = gpu_prefill(dev, h, X, 1)
+            check_routing(B, lay, X, idx, w, 1)
+            ref = np.empty((T, H), np.float64)
+            B.oracle().or_prefill_moe_f64(ref, X, T, C.byref(lay.or_layer()), idx, w)
+            err.append(rel_err(out, ref))
+        assert err[1] < TOL < err[0] < 4 * 2.0 ** -9 + TOL
+    finally:
+        dev.set_bf16sim(0)
         L.ds_hip_layer_destroy(h)
 
 
