@@ -123,10 +123,9 @@ __device__ __forceinline__ u32x4 dsh_load_nt(const void *p) {
 
 // The reference's INT8 row loop in its own order (int8_matvec_generic, ds_quantize.c:163-166, which
 // GCC keeps scalar and contracts): dot = fma(u_j, x_j, dot) for j = 0, 1, ... with the exact code
-// u = q + 128, and with XS also xs += x_j in the same loop. One lane runs one row, so the result
+// u = q + 128, and xs += x_j in the same loop. One lane runs one row, so the result
 // is bit-identical to the reference's. row: 16-byte aligned, n % 16 == 0; x in LDS (the lanes of a
 // wave read the same x_j at once: a broadcast). Loads run PF 16-byte chunks ahead in registers.
-template <bool XS>
 __device__ __forceinline__ float dsh_row_chain(const int8_t *row, const float *x, int n, float &xs) {
   constexpr int PF = 16;
   const int C = n >> 4;
@@ -153,7 +152,7 @@ __device__ __forceinline__ float dsh_row_chain(const int8_t *row, const float *x
 #pragma unroll
           for (int c = 0; c < 4; c++) {
             dot = __builtin_fmaf(u[c], xv[c], dot);
-            if (XS) xs += xv[c];
+            xs += xv[c];
           }
         }
       }

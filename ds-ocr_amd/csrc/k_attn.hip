@@ -491,13 +491,13 @@ __global__ void __launch_bounds__(256) k_attn_av(dsh_attn_t A, const int *pos_pt
 }
 
 // ---------------------------------------------------------------------------- O projection
-// 16 output rows per block (threads past 256 only help with att); every block puts att together itself (head h: the parts' sums times
-// the product of the later parts' corrections, in part order, times 1/sum_e: ds_vec_scale_inplace, sum_e > 0),
-// at most 30 x q_dim floats from L2, which costs less than a launch of its own: 5.7 us in all at 702 positions
-// and 6.6 at 7002, against 5.8 + 3.7 and 5.0 + 9.9 in two kernels. q_dim == 32*N32.
+// 16 output rows per block (threads past 256 only help with att); every block puts att together itself (head h: the
+// parts' sums times the product of the later parts' corrections, in part order, times 1/sum_e: ds_vec_scale_inplace,
+// sum_e > 0), at most 30 x q_dim floats from L2, which costs less than a launch of its own: 5.7 us in all at 702
+// positions and 6.6 at 7002, against 5.8 + 3.7 and 5.0 + 9.9 in two kernels. q_dim == 32*N32.
 template <int N32>
-__global__ void __launch_bounds__(attn_threads(32 * N32)) k_attn_oproj(dsh_attn_t A, const int *pos_ptr, int pos_add, int prefill_len,
-                                                    int window, int chunk) {
+__global__ void __launch_bounds__(attn_threads(32 * N32))
+    k_attn_oproj(dsh_attn_t A, const int *pos_ptr, int pos_add, int prefill_len, int window, int chunk) {
   constexpr int QD = 32 * N32, PP = 16;  // parts in flight
   __shared__ __attribute__((aligned(16))) float s_a[QD];
   __shared__ float s_f[QD / 64 * DSH_ATTN_PARTS], s_inv[QD / 64];

@@ -168,7 +168,7 @@ __global__ void __launch_bounds__(256) k_int8_matvec_chain(const int8_t *__restr
   const int8_t *qr = q + (size_t)r * in_dim;
   float dot, xs = 0.0f;
   if (ALIGNED) {
-    dot = dsh_row_chain<true>(qr, s_x, in_dim, xs);
+    dot = dsh_row_chain(qr, s_x, in_dim, xs);
   } else {
     dot = 0.0f;
     for (int c = 0; c < in_dim; c++) {
@@ -865,10 +865,11 @@ __global__ void __launch_bounds__(256) k_sum_pairs_f64(const double *__restrict_
 // Y[M,N] = X[M,K] * W[N,K]^T with W widened from bf16 (ds_linear_nobias_bf16, seq_len > 1: the
 // reference converts W to f32 and calls sgemm, ds_kernels.c:917-927), on the bf16 MFMA: x is split into three bf16
 // numbers of 8 bits each, x = x1 + x2 + x3 exactly for |x| >= 2^-103 (below, the parts run into bf16's subnormal grid,
-// and from 2^-110 on lose bits), so every product w x_i is exact in f32 and only the sums round, 32 columns to an MFMA step instead of one to a fused multiply-add (error against f64 at K = 1280: 2.1e-7 relative,
-// 6.4e-7 for the chain of fused multiply-adds). A block of 4 waves takes 64 x 64 of Y, a wave 32 x 32; K runs in
-// stages of 64 columns, split on their way into LDS (rows of 72 elements: 16-byte reads of 16 rows spread over
-// all banks), the next stage on its way in registers. At 662 x 1280 x 1280 (220 blocks) bound by the 20 stages'
+// and from 2^-110 on lose bits), so every product w x_i is exact in f32 and only the sums round, 32 columns to an MFMA
+// step instead of one to a fused multiply-add (error against f64 at K = 1280: 2.1e-7 relative, 6.4e-7 for the chain of
+// fused multiply-adds). A block of 4 waves takes 64 x 64 of Y, a wave 32 x 32; K runs in stages of 64 columns, split
+// on their way into LDS (rows of 72 elements: 16-byte reads of 16 rows spread over all banks), the next stage on its
+// way in registers. At 662 x 1280 x 1280 (220 blocks) bound by the 20 stages'
 // latency: 28.7 us, 227 us for scalar f32 tiles. VEC: K % 8 == 0 (16-byte loads of both operands' rows).
 // A tile with a smaller x other than zero in its rows goes through gb_tile_fma, 8 times as slow; looking for one costs
 // 0.9 us of a kernel at K = 1280 (two instructions per element, one more reduction over the block).

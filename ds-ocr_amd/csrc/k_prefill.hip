@@ -16,9 +16,11 @@
 // Kernels (one launch each, all sizes fixed by T, so a graph can hold them):
 //   k_pf_route_cfg  CFG: per token, the router scores in ds_linear's order, x → the two int8 limbs
 //                and their scale, Σx; expert selection → idx, w
-//   k_pf_scores_bf16, k_pf_select_dec  DECODE: the bf16 router's scores in the reference's AVX-512
-//                order, then the limbs and the selection
-//   k_pf_plan    expert-sorted (token, slot) pairs, per-expert offsets and the GEMM work items (expert, up-to-PF_MT-row chunk)
+//   k_pf_scores_bf16, _bf16r, _mfma  DECODE: the bf16 router's scores in the reference's AVX-512 order (any row path;
+//                the rows in registers; on the f32 MFMA: pf_scores_kind chooses)
+//   k_pf_select_dec  DECODE: the limbs and the selection
+//   k_pf_plan    expert-sorted (token, slot) pairs, per-expert offsets, the GEMM work items (expert, up-to-PF_MT-row
+//                chunk) and k_pf_moe's queues
 //   k_pf_gate_up grouped GEMM + SwiGLU → h as limbs, its per-(row, n-tile) sums and maxima, for
 //                routed pairs and for the shared expert
 //   k_pf_down    grouped GEMM → Y (f32) per routed pair and per token for the shared expert
@@ -35,8 +37,10 @@ typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 #define PF_MT 64      // A rows per work item
-#define PF_EU 128     // intermediate units that share a limb exponent in a row of h
-#define PF_NT_MAX 16  // such groups per row of h (I, SI <= 2048)
+#define PF_NB 4       // 16-row n-blocks of weights per wave of a GEMM tile
+#define PF_EU 128     // intermediate units of a gate_up tile, which share a limb exponent in a row of h (32 per wave)
+#define PF_DN 256     // output rows of a down tile (64 per wave)
+#define PF_NT_MAX 16  // gate_up tiles per row of h (I, SI <= 2048)
 #define PF_TB 8     // tokens per DECODE-mode scores block
 #define PF_PLAN_LDS 65536  // (token, slot) entries the plan kernel caches in LDS (a byte each)
 #define PF_NQ 8           // work queues of the fused GEMM kernel: one per XCD
@@ -371,8 +375,10 @@ __global__ void __launch_bounds__(256) k_pf_scores_bf16r(const uint16_t *__restr
 // MFMAs over its columns. A block takes 16 tokens x 64 experts; wave v runs chains 8v .. 8v+7 (columns
 // 32i + 8v + c), four 16-expert blocks per instruction, 16 accumulators per chain and lane. Router rows and
 // tokens pass through LDS 128 columns at a time (swizzled 16-byte pieces), the next ones on their way in registers.
-// Then the order's own sums: a0 + a1 (waves 0 + 2, 1 + 3), T3 (waves 0 + 1), T6 and the last pair.
-// 18.5 us at 3001 tokens; k_pf_scores_bf16r, which unpacks a row and reads x from LDS for every token, takes 46.5.
+// Then the order's own sums: a0 + a1 (waves 0 + 2, 1 + 3), T3 (waves 0 + 1), T6 and the last pair. Scores, products and
+// inputs down to 2^-149 give k_pf_scores_bf16's bits (compared at H 256, 512 and 1280).
+// 16.6 us at 3001 tokens x 1280; k_pf_scores_bf16r, which unpacks a row and reads x from LDS for every token, takes
+// 43.4. 128 accumulators and the operands come to 256 registers, and 12 spill (52 bytes of scratch per lane).
 #define PF_SM_T 16
 struct pf_scores_smem {
   union {
@@ -517,8 +523,8 @@ __global__ void __launch_bounds__(256) k_pf_select_dec(const float *__restrict__
 
 // ---------------------------------------------------------------------------------- plan
 // One 1024-thread block. Its time is a chain of round trips (5-8 us up to 662 tokens): the entries come from memory once
-// (a byte each in LDS: read again from memory for each 64 they took 16 of 24 us at 3001 tokens). Wave v owns a contiguous range of the T·K (token, slot) entries. Per-wave
-// expert counts give each expert's segment offset and each wave's start inside it, so a pair's
+// (a byte each in LDS: read again from memory for each 64 they took 16 of 24 us at 3001 tokens). Wave v owns a
+// contiguous range of the T·K (token, slot) entries. Per-wave expert counts give each expert's segment offset and each wave's start inside it, so a pair's
 // position is (segment offset) + (pairs of the expert in earlier waves) + (earlier pairs of the
 // expert in this wave). Entries with no expert (idx < 0 or >= E) get pos_of = -1.
 // Work items: each expert's pairs in chunks of PF_MT (items 0 .. n_routed-1), then the shared
@@ -775,29 +781,20 @@ static_assert(PF_EU == PF_KS, "the down main loop takes one exponent of h per ro
 #define PF_OCC 2  // GEMM blocks per CU the register budget is sized for
 #endif
 
-// Tile shape: up to MT A rows, NB 16-row n-blocks per wave. GU intermediate units (their gate and up rows) per
-// gate_up tile, DN output rows per down tile.
-template <int MT_, int NB_>
-struct pf_shape {
-  static constexpr int MT = MT_, NB = NB_, GU = 32 * NB_, DN = 64 * NB_;
-};
-typedef pf_shape<PF_MT, 4> pf_tile_t;
-
-template <typename C>
 struct pf_smem {
   union {
     struct {
-      int8_t A[2][2][C::MT][PF_KS];  // [stage parity][low, high limb][row][column, swizzled]
+      int8_t A[2][2][PF_MT][PF_KS];  // [stage parity][low, high limb][row][column, swizzled]
     } q;                             // main loop
-    float red[4][C::MT][8 * C::NB + 1];  // gate_up epilogue: h values per wave
+    float red[4][PF_MT][8 * PF_NB + 1];  // gate_up epilogue: h values per wave
   } u;
-  float hsum[4][C::MT];  // Σh of the block's A rows (gate_up: per wave)
-  float hmx[4][C::MT];   // gate_up: max |h| of the block's A rows, per wave
-  float xs[C::MT];       // gate_up: Σx of the block's A rows (their tokens)
-  float xsc[C::MT];      // the A rows' limb scale 2^(e-15)
-  short ek[C::MT][PF_NT_MAX];  // down: exponent of each A row's unit groups
-  float hp[C::MT][PF_NT_MAX];  // down: Σh of each A row's unit groups (the gate_up partials)
-  int erow[C::MT];             // down: the A rows' common exponent (max over their groups)
+  float hsum[4][PF_MT];  // Σh of the block's A rows (gate_up: per wave)
+  float hmx[4][PF_MT];   // gate_up: max |h| of the block's A rows, per wave
+  float xs[PF_MT];       // gate_up: Σx of the block's A rows (their tokens)
+  float xsc[PF_MT];      // the A rows' limb scale 2^(e-15)
+  short ek[PF_MT][PF_NT_MAX];  // down: exponent of each A row's n-tiles
+  float hp[PF_MT][PF_NT_MAX];  // down: Σh of each A row's n-tiles (the gate_up partials)
+  int erow[PF_MT];             // down: the A rows' common exponent (max over their n-tiles)
 };
 
 // Limb exponent of a set of values with max |v| = mx: 2^e > mx·(1 + 2^-7), so rint(v·2^(15-e)) + 128
@@ -907,8 +904,8 @@ hipError_t dsh_launch_pf_swiglu_check(unsigned long long *counts, hipStream_t s)
 // distinct bank groups, and two consecutive rows fill 256 contiguous bytes
 __device__ __forceinline__ int pf_swz(int r) { return (r ^ (r >> 3)) & 7; }
 
-// Stages of loads in flight per wave (what the registers allow beside 32 MB accumulators): A and B registers of a stage are reloaded with the stage D later once they
-// are used. A wave's loads return in issue order, so A runs as far ahead as B: an A stage loaded one
+// Stages of loads in flight per wave (what the registers allow beside 32 MB accumulators): A and B registers of a stage
+// are reloaded with the stage D later once they are used. A wave's loads return in issue order, so A runs as far ahead as B: an A stage loaded one
 // stage ahead would wait for every weight load issued before it.
 constexpr int pf_depth(int MB) { return MB == 1 ? 3 : (MB == 2 ? 2 : 1); }
 
@@ -926,8 +923,8 @@ constexpr int pf_depth(int MB) { return MB == 1 ? 3 : (MB == 2 ? 2 : 1); }
 // register i holds A row 16mb + 4(l/16) + i, weight row 16j + l%16. A rows past the item's count
 // repeat a valid row; their results are never stored.
 // A is two int8 limb arrays, A0 low and A1 high (gate_up: x at one exponent per row; down: h at
-// one exponent per row and 64-column half stage). ALIGN (down): before a stage's A values go to LDS,
-// each is brought to its row's common exponent (pf_align16 with d = erow - ek of the row's half stage;
+// one exponent per row and 128-column stage, a gate_up tile's units). ALIGN (down): before a stage's A values go to
+// LDS, each is brought to its row's common exponent (pf_align16 with d = erow - ek of the row's stage;
 // sm.ek, sm.erow; trow: the table rows of this thread's A rows).
 // pre() runs once the first stages' loads are issued (down: building the alignment table), so its
 // waits leave them in flight.
@@ -939,11 +936,11 @@ struct pf_arows {  // A rows a thread copies: pf_arow(c), c < N (MB 1: two threa
   }
 };
 
-template <typename C, int MB, bool ALIGN, typename Pre>
+template <int MB, bool ALIGN, typename Pre>
 __device__ __forceinline__ void pf_mainloop_i8(const int8_t *A0, const int8_t *A1, const size_t *arow,
                                                const int *trow, int K, const int8_t *brow0, const int8_t *brow1,
-                                               i32x4 (&acc)[MB][C::NB][2], pf_smem<C> &sm, Pre &&pre) {
-  constexpr int NB = C::NB, D = pf_depth(MB), NA = pf_arows<MB>::N;
+                                               i32x4 (&acc)[MB][PF_NB][2], pf_smem &sm, Pre &&pre) {
+  constexpr int NB = PF_NB, D = pf_depth(MB), NA = pf_arows<MB>::N;
   const int lane = threadIdx.x & 63, r16 = lane & 15, kg = lane >> 4;
   const int ac = threadIdx.x & 7;  // A copy: chunk ac of the thread's rows
   const int nk = K / PF_KS;
@@ -1044,19 +1041,19 @@ __device__ __forceinline__ float pf_row16_max(float v) {  // over each aligned g
   return fmaxf(v, dsh_dpp<0x140>(v));
 }
 
-// gate_up: block = (work item, n-tile): the item's A rows (tokens) x GU intermediate units; wave w
-// owns the 16·NB/2 units from i0 + 16·NB/2·w: its first NB/2 n-blocks are their gate rows, the others their up rows,
-// so each SwiGLU pair sits in the same lane and register (n-blocks h and NB/2 + h).
-template <typename C, bool SHARED, int MB>
+// gate_up: block = (work item, n-tile): the item's A rows (tokens) x PF_EU intermediate units; wave w
+// owns units i0 + 32w .. +31: n-blocks 0, 1 = their gate rows, 2, 3 = their up rows, so each SwiGLU
+// pair sits in the same lane and register (n-blocks h and 2 + h).
+template <bool SHARED, int MB>
 __device__ __forceinline__ void gate_up_tile(const dsh_layer_t &L, const pf_item &it, int nt, const int8_t *X0,
                                              const int8_t *X1, const float *xsc, const float *xsum,
                                              const int *pair_tok, int bf16sim, int8_t *Hq0, int8_t *Hq1,
-                                             float *hpart, float *hmaxp, pf_smem<C> &sm) {
-  constexpr int HB = C::NB / 2, WU = 16 * HB, WG = PF_EU / WU;  // 16-unit blocks and units per wave, waves per group
+                                             float *hpart, float *hmaxp, pf_smem &sm) {
+  constexpr int HB = PF_NB / 2, WU = 16 * HB;  // 16-unit blocks and units per wave
   const int H = L.H;
   const int Iseg = SHARED ? L.SI : L.I, ntK = Iseg / PF_EU;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r16 = lane & 15, kg = lane >> 4;
-  const int u0 = nt * C::GU + wave * WU;
+  const int u0 = nt * PF_EU + wave * WU;
   const int8_t *wq = SHARED ? L.sgu_q : L.gu_q + (size_t)it.seg * 2 * L.I * H;
   const float *wso = SHARED ? L.sgu_so : L.gu_so + (size_t)it.seg * 2 * L.I * 2;
   constexpr int NA = pf_arows<MB>::N;
@@ -1088,8 +1085,8 @@ __device__ __forceinline__ void gate_up_tile(const dsh_layer_t &L, const pf_item
     sog[h] = ((const float2 *)wso)[unit];
     sou[h] = ((const float2 *)wso)[Iseg + unit];
   }
-  i32x4 acc[MB][C::NB][2];
-  pf_mainloop_i8<C, MB, false>(X0, X1, arow, nullptr, H, wq + (size_t)u0 * H, wq + (size_t)(Iseg + u0) * H, acc, sm,
+  i32x4 acc[MB][PF_NB][2];
+  pf_mainloop_i8<MB, false>(X0, X1, arow, nullptr, H, wq + (size_t)u0 * H, wq + (size_t)(Iseg + u0) * H, acc, sm,
                                [] {});
   // signed codes: offset + 128·scale multiplies Σa
 #pragma unroll
@@ -1099,9 +1096,9 @@ __device__ __forceinline__ void gate_up_tile(const dsh_layer_t &L, const pf_item
   }
   const size_t rbase = SHARED ? (size_t)it.m0 : (size_t)(it.pos0 + it.m0);
   // The tile's h values go to LDS (per wave: its rows x its units); the sums and maxima over a row's units run
-  // by DPP over the 16 lanes that hold them, then over the waves of a group of PF_EU units, whose maximum gives
-  // the group's limb exponent; the lanes then store 8-unit runs of both limbs.
-  float(*red)[C::MT][8 * C::NB + 1] = sm.u.red;
+  // by DPP over the 16 lanes that hold them, then over the waves; a row's maximum over the tile's PF_EU units gives
+  // its limb exponent there; the lanes then store 8-unit runs of both limbs.
+  float(*red)[PF_MT][8 * PF_NB + 1] = sm.u.red;
   __syncthreads();  // every wave is done with the main loop's tiles
   // rows past the item's count repeat row 0 (valid values, never stored); the bf16 simulation is
   // one branch around the loop
@@ -1143,12 +1140,7 @@ __device__ __forceinline__ void gate_up_tile(const dsh_layer_t &L, const pf_item
   else
     h_out(std::false_type{});
   __syncthreads();
-  auto group_max = [&](int g, int m) {
-    float mx = sm.hmx[g * WG][m];
-#pragma unroll
-    for (int w = 1; w < WG; w++) mx = fmaxf(mx, sm.hmx[g * WG + w][m]);
-    return mx;
-  };
+  auto row_max = [&](int m) { return fmaxf(fmaxf(fmaxf(sm.hmx[0][m], sm.hmx[1][m]), sm.hmx[2][m]), sm.hmx[3][m]); };
   {  // stores: lane → row lane / LR + (64 / LR)·k, units 8·(lane % LR) .. +7 of the wave's, as limbs
     constexpr int LR = WU / 8, RP = 64 / LR;
     const int g8 = 8 * (lane % LR);
@@ -1156,7 +1148,7 @@ __device__ __forceinline__ void gate_up_tile(const dsh_layer_t &L, const pf_item
     for (int k = 0; k < (16 * MB + RP - 1) / RP; k++) {
       const int m = lane / LR + RP * k;
       if (m >= it.mcnt) continue;
-      const float f = __builtin_ldexpf(1.0f, 15 - pf_limb_exp(group_max(wave / WG, m)));
+      const float f = __builtin_ldexpf(1.0f, 15 - pf_limb_exp(row_max(m)));
       f32x4 v0, v1;
 #pragma unroll
       for (int i = 0; i < 4; i++) {
@@ -1173,28 +1165,22 @@ __device__ __forceinline__ void gate_up_tile(const dsh_layer_t &L, const pf_item
   }
   if (threadIdx.x < it.mcnt) {
     const int m = threadIdx.x;
-#pragma unroll
-    for (int g = 0; g < C::GU / PF_EU; g++) {
-      float tot = sm.hsum[g * WG][m];
-#pragma unroll
-      for (int w = 1; w < WG; w++) tot += sm.hsum[g * WG + w][m];
-      hpart[(rbase + m) * ntK + nt * (C::GU / PF_EU) + g] = tot;
-      hmaxp[(rbase + m) * ntK + nt * (C::GU / PF_EU) + g] = group_max(g, m);
-    }
+    hpart[(rbase + m) * ntK + nt] = ((sm.hsum[0][m] + sm.hsum[1][m]) + sm.hsum[2][m]) + sm.hsum[3][m];
+    hmaxp[(rbase + m) * ntK + nt] = row_max(m);
   }
 }
 
-template <typename C, bool SHARED>
+template <bool SHARED>
 __device__ __forceinline__ void gate_up_dispatch(const dsh_layer_t &L, const pf_item &it, int nt, const int8_t *X0,
                                                  const int8_t *X1, const float *xsc, const float *xsum,
                                                  const int *pair_tok, int bf16sim, int8_t *Hq0, int8_t *Hq1,
-                                                 float *hpart, float *hmaxp, pf_smem<C> &sm) {
+                                                 float *hpart, float *hmaxp, pf_smem &sm) {
   if (it.mcnt <= 16)
-    gate_up_tile<C, SHARED, 1>(L, it, nt, X0, X1, xsc, xsum, pair_tok, bf16sim, Hq0, Hq1, hpart, hmaxp, sm);
+    gate_up_tile<SHARED, 1>(L, it, nt, X0, X1, xsc, xsum, pair_tok, bf16sim, Hq0, Hq1, hpart, hmaxp, sm);
   else if (it.mcnt <= 32)
-    gate_up_tile<C, SHARED, 2>(L, it, nt, X0, X1, xsc, xsum, pair_tok, bf16sim, Hq0, Hq1, hpart, hmaxp, sm);
+    gate_up_tile<SHARED, 2>(L, it, nt, X0, X1, xsc, xsum, pair_tok, bf16sim, Hq0, Hq1, hpart, hmaxp, sm);
   else
-    gate_up_tile<C, SHARED, 4>(L, it, nt, X0, X1, xsc, xsum, pair_tok, bf16sim, Hq0, Hq1, hpart, hmaxp, sm);
+    gate_up_tile<SHARED, 4>(L, it, nt, X0, X1, xsc, xsum, pair_tok, bf16sim, Hq0, Hq1, hpart, hmaxp, sm);
 }
 
 __global__ void __launch_bounds__(256, PF_OCC) k_pf_gate_up(dsh_layer_t L, const pf_item *__restrict__ items,
@@ -1205,35 +1191,34 @@ __global__ void __launch_bounds__(256, PF_OCC) k_pf_gate_up(dsh_layer_t L, const
                                                        pf_hq hq, float *__restrict__ hpr, float *__restrict__ hps,
                                                        float *__restrict__ hmr, float *__restrict__ hms,
                                                        const int *__restrict__ tiles) {
-  typedef pf_tile_t C;
-  __shared__ __attribute__((aligned(16))) pf_smem<C> sm;
+  __shared__ __attribute__((aligned(16))) pf_smem sm;
   int item, nt;
-  if (!pf_tile(counts, tiles, L.SI / C::GU, L.I / C::GU, item, nt)) return;
+  if (!pf_tile(counts, tiles, L.SI / PF_EU, L.I / PF_EU, item, nt)) return;
   const pf_item it = items[item];
   if (it.seg == L.E)
-    gate_up_dispatch<C, true>(L, it, nt, X0, X1, xsc, xsum, pair_tok, bf16sim, hq.s0, hq.s1, hps, hms, sm);
+    gate_up_dispatch<true>(L, it, nt, X0, X1, xsc, xsum, pair_tok, bf16sim, hq.s0, hq.s1, hps, hms, sm);
   else
-    gate_up_dispatch<C, false>(L, it, nt, X0, X1, xsc, xsum, pair_tok, bf16sim, hq.r0, hq.r1, hpr, hmr, sm);
+    gate_up_dispatch<false>(L, it, nt, X0, X1, xsc, xsum, pair_tok, bf16sim, hq.r0, hq.r1, hpr, hmr, sm);
 }
 
 // down: block = (work item, n-tile): the item's A rows (h of its pairs, or of tokens for the shared
-// expert, as limbs) x DN output rows; wave w owns 16·NB of them as NB 16-row n-blocks. Each A
-// row's exponent is the largest of its groups' (from the max |h| per (row, group of PF_EU units) the gate_up
-// epilogues wrote; read at L2); the main loop aligns every half stage to it. Σh of each A row is the sum,
-// in group order, of the per-group row sums the gate_up epilogue wrote.
-template <typename C, bool SHARED, int MB>
+// expert, as limbs) x PF_DN output rows; wave w owns rows n0 + 64w .. +63 as four 16-row n-blocks. Each A
+// row's exponent is the largest of its n-tiles' (from the max |h| per (row, gate_up n-tile) the gate_up
+// epilogues wrote; read at L2); the main loop aligns every stage to it. Σh of each A row is the sum,
+// in n-tile order, of the per-n-tile row sums the gate_up epilogue wrote.
+template <bool SHARED, int MB>
 __device__ __forceinline__ void down_tile(const dsh_layer_t &L, const pf_item &it, int nt, const int8_t *Hq0,
                                           const int8_t *Hq1, const float *hpart, const float *hmaxp, float *Y,
-                                          pf_smem<C> &sm) {
-  constexpr int NB = C::NB, NE = 16 * MB * PF_NT_MAX / 256, NA = pf_arows<MB>::N;
+                                          pf_smem &sm) {
+  constexpr int NB = PF_NB, NE = 16 * MB * PF_NT_MAX / 256, NA = pf_arows<MB>::N;
   const int H = L.H;
   const int Kd = SHARED ? L.SI : L.I, ntK = Kd / PF_EU;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r16 = lane & 15, kg = lane >> 4;
   const int8_t *wq = SHARED ? L.sdn_q : L.dn_q + (size_t)it.seg * H * L.I;
   const float *wso = SHARED ? L.sdn_so : L.dn_so + (size_t)it.seg * H * 2;
-  const int nw = nt * C::DN + wave * 16 * NB;
+  const int nw = nt * PF_DN + wave * 16 * NB;
   const size_t rbase = SHARED ? (size_t)it.m0 : (size_t)(it.pos0 + it.m0);
-  // The gate_up partials of the A rows (max |h| and Σh per row and group; at most MB·16 x
+  // The gate_up partials of the A rows (max |h| and Σh per row and n-tile; at most MB·16 x
   // PF_NT_MAX), read at L2 and all issued at once, then the output rows' scales and offsets; all are in flight
   // while the main loop issues its first stages.
   const int ntot = it.mcnt * ntK;
@@ -1251,8 +1236,8 @@ __device__ __forceinline__ void down_tile(const dsh_layer_t &L, const pf_item &i
   float2 so[NB];
 #pragma unroll
   for (int j = 0; j < NB; j++) so[j] = ((const float2 *)wso)[nw + 16 * j + r16];
-  if (threadIdx.x < C::MT) sm.erow[threadIdx.x] = -1024;
-  // each A row's exponent (the largest of its groups'), its limb scale and its Σh (group order)
+  if (threadIdx.x < PF_MT) sm.erow[threadIdx.x] = -1024;
+  // each A row's exponent (the largest of its n-tiles'), its limb scale and its Σh (n-tile order)
   auto table = [&] {
     __syncthreads();
 #pragma unroll
@@ -1283,7 +1268,7 @@ __device__ __forceinline__ void down_tile(const dsh_layer_t &L, const pf_item &i
     arow[c] = (rbase + trow[c]) * Kd;
   }
   i32x4 acc[MB][NB][2];
-  pf_mainloop_i8<C, MB, true>(Hq0, Hq1, arow, trow, Kd, wq + (size_t)nw * Kd, wq + (size_t)(nw + 8 * NB) * Kd, acc,
+  pf_mainloop_i8<MB, true>(Hq0, Hq1, arow, trow, Kd, wq + (size_t)nw * Kd, wq + (size_t)(nw + 8 * NB) * Kd, acc,
                               sm, table);
 #pragma unroll
   for (int j = 0; j < NB; j++) {
@@ -1303,16 +1288,16 @@ __device__ __forceinline__ void down_tile(const dsh_layer_t &L, const pf_item &i
   }
 }
 
-template <typename C, bool SHARED>
+template <bool SHARED>
 __device__ __forceinline__ void down_dispatch(const dsh_layer_t &L, const pf_item &it, int nt, const int8_t *Hq0,
                                               const int8_t *Hq1, const float *hpart, const float *hmaxp, float *Y,
-                                              pf_smem<C> &sm) {
+                                              pf_smem &sm) {
   if (it.mcnt <= 16)
-    down_tile<C, SHARED, 1>(L, it, nt, Hq0, Hq1, hpart, hmaxp, Y, sm);
+    down_tile<SHARED, 1>(L, it, nt, Hq0, Hq1, hpart, hmaxp, Y, sm);
   else if (it.mcnt <= 32)
-    down_tile<C, SHARED, 2>(L, it, nt, Hq0, Hq1, hpart, hmaxp, Y, sm);
+    down_tile<SHARED, 2>(L, it, nt, Hq0, Hq1, hpart, hmaxp, Y, sm);
   else
-    down_tile<C, SHARED, 4>(L, it, nt, Hq0, Hq1, hpart, hmaxp, Y, sm);
+    down_tile<SHARED, 4>(L, it, nt, Hq0, Hq1, hpart, hmaxp, Y, sm);
 }
 
 __global__ void __launch_bounds__(256, PF_OCC) k_pf_down(dsh_layer_t L, const pf_item *__restrict__ items,
@@ -1321,15 +1306,14 @@ __global__ void __launch_bounds__(256, PF_OCC) k_pf_down(dsh_layer_t L, const pf
                                                     const float *__restrict__ hmr, const float *__restrict__ hms,
                                                     float *__restrict__ Y, float *__restrict__ Ysh,
                                                     const int *__restrict__ tiles) {
-  typedef pf_tile_t C;
-  __shared__ __attribute__((aligned(16))) pf_smem<C> sm;
+  __shared__ __attribute__((aligned(16))) pf_smem sm;
   int item, nt;
-  if (!pf_tile(counts, tiles, L.H / C::DN, L.H / C::DN, item, nt)) return;
+  if (!pf_tile(counts, tiles, L.H / PF_DN, L.H / PF_DN, item, nt)) return;
   const pf_item it = items[item];
   if (it.seg == L.E)
-    down_dispatch<C, true>(L, it, nt, hq.s0, hq.s1, hps, hms, Ysh, sm);
+    down_dispatch<true>(L, it, nt, hq.s0, hq.s1, hps, hms, Ysh, sm);
   else
-    down_dispatch<C, false>(L, it, nt, hq.r0, hq.r1, hpr, hmr, Y, sm);
+    down_dispatch<false>(L, it, nt, hq.r0, hq.r1, hpr, hmr, Y, sm);
 }
 
 // Fused grouped GEMM: one launch runs every gate_up and down tile, one tile per block. A block
@@ -1353,8 +1337,7 @@ __global__ void __launch_bounds__(256, PF_OCC) k_pf_moe(dsh_layer_t L, const pf_
                                                     int bf16sim, pf_hq hq, float *hpr, float *hps, float *hmr,
                                                     float *hms, float *__restrict__ Y,
                                                     float *__restrict__ Ysh) {
-  typedef pf_tile_t C;
-  __shared__ __attribute__((aligned(16))) pf_smem<C> sm;
+  __shared__ __attribute__((aligned(16))) pf_smem sm;
   __shared__ int s_tile;
   unsigned xcc;
   asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(xcc));
@@ -1368,15 +1351,15 @@ __global__ void __launch_bounds__(256, PF_OCC) k_pf_moe(dsh_layer_t L, const pf_
   const pf_item it = items[item];
   if (!(d & PF_DN_TILE)) {
     if (it.seg == L.E)
-      gate_up_dispatch<C, true>(L, it, nt, X0, X1, xsc, xsum, pair_tok, bf16sim, hq.s0, hq.s1, hps, hms, sm);
+      gate_up_dispatch<true>(L, it, nt, X0, X1, xsc, xsum, pair_tok, bf16sim, hq.s0, hq.s1, hps, hms, sm);
     else
-      gate_up_dispatch<C, false>(L, it, nt, X0, X1, xsc, xsum, pair_tok, bf16sim, hq.r0, hq.r1, hpr, hmr, sm);
+      gate_up_dispatch<false>(L, it, nt, X0, X1, xsc, xsum, pair_tok, bf16sim, hq.r0, hq.r1, hpr, hmr, sm);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this thread's limb and partial stores are in L2
     __syncthreads();
     if (threadIdx.x == 0) __hip_atomic_fetch_add(Q.gu_done + item, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   } else {
     if (threadIdx.x == 0) {
-      const int need = it.seg == L.E ? L.SI / C::GU : L.I / C::GU;
+      const int need = it.seg == L.E ? L.SI / PF_EU : L.I / PF_EU;
       int spins = 0;
       bool gave_up = Q.spin_max < 0;
       while (!gave_up && __hip_atomic_load(Q.gu_done + item, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < need) {
@@ -1390,9 +1373,9 @@ __global__ void __launch_bounds__(256, PF_OCC) k_pf_moe(dsh_layer_t L, const pf_
     }
     __syncthreads();
     if (it.seg == L.E)
-      down_dispatch<C, true>(L, it, nt, hq.s0, hq.s1, hps, hms, Ysh, sm);
+      down_dispatch<true>(L, it, nt, hq.s0, hq.s1, hps, hms, Ysh, sm);
     else
-      down_dispatch<C, false>(L, it, nt, hq.r0, hq.r1, hpr, hmr, Y, sm);
+      down_dispatch<false>(L, it, nt, hq.r0, hq.r1, hpr, hmr, Y, sm);
   }
 }
 
@@ -1510,8 +1493,8 @@ struct pf_ws {
   pf_hq hq;         // SwiGLU outputs h as int8 limbs: routed [TK][I], shared [T][SI]
   float *Y, *Ysh;
   float *ps;        // [T][4][64] router scores (DECODE: the full score in row 0, rows 1-3 zero)
-  float *hpr, *hps; // Σh partials per (row, group of 64 units): routed [TK][I/64], shared [T][SI/64]
-  float *hmr, *hms; // max |h| per (row, group), same layout
+  float *hpr, *hps; // Σh partials per (row, gate_up n-tile): routed [TK][I/128], shared [T][SI/128]
+  float *hmr, *hms; // max |h| per (row, gate_up n-tile), same layout
   int *tiles_gu, *tiles_dn;  // routed GEMM tiles (item << 8 | n-tile) in launch order
   int *qtiles, *qcount, *qnext, *gu_done, *err;  // fused kernel: work queues, counters, wait error
 };
@@ -1530,7 +1513,7 @@ int pf_grid(const dsh_layer_t *L, int T, int ntS, int ntR) {
 // Tiles one fused-kernel queue can hold: every gate_up and down tile of the largest work list.
 size_t pf_queue_cap(const dsh_layer_t *L, int T) {
   const size_t r = pf_max_routed_items(L, T), sh = pf_shared_items(T);
-  return r * (L->I / pf_tile_t::GU) + sh * (L->SI / pf_tile_t::GU) + (r + sh) * (L->H / pf_tile_t::DN);
+  return r * (L->I / PF_EU) + sh * (L->SI / PF_EU) + (r + sh) * (L->H / PF_DN);
 }
 
 // Blocks per XCD of the fused launch, at least the tiles of the longest queue: its cost is at most the mean and the
@@ -1538,7 +1521,7 @@ size_t pf_queue_cap(const dsh_layer_t *L, int T) {
 // items of one expert), and a tile costs at least the smaller of the kinds' means.
 long pf_queue_blocks(const dsh_layer_t *L, int T) {
   const int nr = pf_max_routed_items(L, T), ns = pf_shared_items(T);
-  const int ngu_r = L->I / pf_tile_t::GU, ngu_s = L->SI / pf_tile_t::GU, ndn = L->H / pf_tile_t::DN;
+  const int ngu_r = L->I / PF_EU, ngu_s = L->SI / PF_EU, ndn = L->H / PF_DN;
   const long cost_r = (long)ngu_r * (L->H / PF_KS) + (long)ndn * (L->I / PF_KS);
   const long cost_s = (long)ngu_s * (L->H / PF_KS) + (long)ndn * (L->SI / PF_KS);
   const long unit = max(cost_s, pf_unit_items(T) * cost_r);
@@ -1600,8 +1583,8 @@ size_t pf_carve(const dsh_layer_t *L, int T, void *base, pf_ws *w) {
   TAKE(hps, float, (size_t)T * (SI / PF_EU));
   TAKE(hmr, float, TK * (I / PF_EU));
   TAKE(hms, float, (size_t)T * (SI / PF_EU));
-  TAKE(tiles_gu, int, (size_t)pf_max_routed_items(L, T) * (I / pf_tile_t::GU));
-  TAKE(tiles_dn, int, (size_t)pf_max_routed_items(L, T) * (H / pf_tile_t::DN));
+  TAKE(tiles_gu, int, (size_t)pf_max_routed_items(L, T) * (I / PF_EU));
+  TAKE(tiles_dn, int, (size_t)pf_max_routed_items(L, T) * (H / PF_DN));
   TAKE(qtiles, int, (size_t)PF_NQ * pf_queue_cap(L, T));
   TAKE(qcount, int, PF_NQ);
   TAKE(qnext, int, PF_NQ);
@@ -1749,19 +1732,19 @@ hipError_t dsh_launch_prefill(const dsh_layer_t *L, const float *X, int T, int r
   const int n_items_max = pf_max_routed_items(L, T) + pf_shared_items(T);
   const bool fused = g_pf_fused == 1 && n_items_max < (1 << 22);
   pf_queues Q{w.qtiles, w.qcount, w.qnext, w.gu_done, w.err, derr, spin_max, (int)pf_queue_cap(L, T),
-              L->I / pf_tile_t::GU, L->SI / pf_tile_t::GU,
-              H / pf_tile_t::DN, H / PF_KS, L->I / PF_KS, L->SI / PF_KS, fused ? 1 : 0};
-  k_pf_plan<<<1, 1024, 0, s>>>(w.idx, T, K, E, L->I / pf_tile_t::GU, H / pf_tile_t::DN, w.seg_off, w.items, w.counts,
+              L->I / PF_EU, L->SI / PF_EU,
+              H / PF_DN, H / PF_KS, L->I / PF_KS, L->SI / PF_KS, fused ? 1 : 0};
+  k_pf_plan<<<1, 1024, 0, s>>>(w.idx, T, K, E, L->I / PF_EU, H / PF_DN, w.seg_off, w.items, w.counts,
                                w.tiles_gu, w.tiles_dn, w.pair_tok, w.pos_of, Q);
   if (fused) {
     const int blocks = (int)(PF_NQ * pf_queue_blocks(L, T));
     k_pf_moe<<<blocks, 256, 0, s>>>(*L, w.items, Q, w.X0, w.X1, w.xsc, w.xsum, w.pair_tok, bf16sim, w.hq, w.hpr,
                                     w.hps, w.hmr, w.hms, w.Y, w.Ysh);
   } else {
-    k_pf_gate_up<<<pf_grid(L, T, L->SI / pf_tile_t::GU, L->I / pf_tile_t::GU), 256, 0, s>>>(
+    k_pf_gate_up<<<pf_grid(L, T, L->SI / PF_EU, L->I / PF_EU), 256, 0, s>>>(
         *L, w.items, w.counts, w.X0, w.X1, w.xsc, w.xsum, w.pair_tok, bf16sim, w.hq, w.hpr, w.hps, w.hmr, w.hms,
         w.tiles_gu);
-    k_pf_down<<<pf_grid(L, T, H / pf_tile_t::DN, H / pf_tile_t::DN), 256, 0, s>>>(*L, w.items, w.counts, w.hq, w.hpr, w.hps,
+    k_pf_down<<<pf_grid(L, T, H / PF_DN, H / PF_DN), 256, 0, s>>>(*L, w.items, w.counts, w.hq, w.hpr, w.hps,
                                                                        w.hmr, w.hms, w.Y, w.Ysh, w.tiles_dn);
   }
   k_pf_combine<<<T, 256, 0, s>>>(X, w.idx, w.w, w.pos_of, w.Y, w.Ysh, H, K, residual, bf16sim, out);
