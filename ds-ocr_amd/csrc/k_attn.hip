@@ -177,7 +177,7 @@ __host__ __device__ constexpr int attn_threads(int n) { return n / 4 > 256 ? n /
 // 16 rows of one of q, k, v per 256-thread block (16 lanes per row): 240 blocks at 1280 x 1280, about one
 // per CU, each with 40 KB of rows in flight behind its input. The rows of a q or k block are eight
 // (d, d + head_dim/2) pairs of one head, a pair in one wave, so the block applies RoPE itself (without the per-head
-// norms, which need the whole head first: then q and k go out as they are, for k_attn_scores). 5.5 us at
+// norms, which need the whole head first: then q and k go out as they are, for k_attn_scores). 5.3 us at
 // 1280 x 1280 (9.8 MB, half of it launch and the input's round trip) against 8.1 with 64 rows per block on 60 CUs.
 // H == 32*N32; head_dim % 16 == 0.
 template <int N32, int NC>
@@ -327,7 +327,7 @@ __device__ void attn_rope_head(const dsh_attn_t &A, int h, int pos, float *s_q, 
 // 0, 2, 1, 3, so that lanes c and c ^ 8 hold the first pairs, and after that add the values repeat as the
 // rotation by 4 needs.
 // NORM: the block norms and ropes q and k itself, and the one that holds the token's own position
-// writes its k into the cache row pos. 3.4 us at 702 positions, 7.5 at 7002 (36 MB, 4.8 TB/s); one thread per
+// writes its k into the cache row pos. 3.5 us at 702 positions, 8.5 at 7002 (36 MB, 4.2 TB/s); one thread per
 // position (a row of 512 bytes per lane) took 5.7 and 13.5.
 template <int HD, bool NORM>
 __global__ void __launch_bounds__(256) k_attn_scores(dsh_attn_t A, const int *pos_ptr, int pos_add, int prefill_len,
@@ -393,7 +393,7 @@ __global__ void __launch_bounds__(256) k_attn_scores(dsh_attn_t A, const int *po
 // max_s = -1e30), a = its correction on a new maximum (else 1), g = 1 on a new maximum (else the weight),
 // c = g * (the product of the later corrections of the chunk). Then every thread adds c * v for 4 dimensions
 // of 1024/HD-th of the positions, its loads issued before the coefficients are known, and the block writes
-// its sum, its sum of c and its product of corrections. 3.8 us at 702 positions, 8.3 at 7002 (36 MB), against 8.9
+// its sum, its sum of c and its product of corrections. 4.0 us at 702 positions, 8.5 at 7002 (36 MB), against 8.9
 // and 25.7 for a kernel with one block per head for the coefficients and one for the sums.
 template <int HD>
 __global__ void __launch_bounds__(256) k_attn_av(dsh_attn_t A, const int *pos_ptr, int pos_add, int prefill_len,
@@ -493,8 +493,8 @@ __global__ void __launch_bounds__(256) k_attn_av(dsh_attn_t A, const int *pos_pt
 // ---------------------------------------------------------------------------- O projection
 // 16 output rows per block (threads past 256 only help with att); every block puts att together itself (head h: the
 // parts' sums times the product of the later parts' corrections, in part order, times 1/sum_e: ds_vec_scale_inplace,
-// sum_e > 0), at most 30 x q_dim floats from L2, which costs less than a launch of its own: 5.7 us in all at 702
-// positions and 6.6 at 7002, against 5.8 + 3.7 and 5.0 + 9.9 in two kernels. q_dim == 32*N32.
+// sum_e > 0), at most 30 x q_dim floats from L2, which costs less than a launch of its own: 5.6 us in all at 702
+// positions and 7.1 at 7002, against 5.8 + 3.7 and 5.0 + 9.9 in two kernels. q_dim == 32*N32.
 template <int N32>
 __global__ void __launch_bounds__(attn_threads(32 * N32))
     k_attn_oproj(dsh_attn_t A, const int *pos_ptr, int pos_add, int prefill_len, int window, int chunk) {
